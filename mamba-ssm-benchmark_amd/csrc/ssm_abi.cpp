@@ -617,22 +617,12 @@ int ssm_lscan_bwd(const ssm_lscan_bwd_args *a, void *stream) {
   p.a = kv(a->a);
   p.b = kv(a->dh);
   p.h = kv(a->db);
+  p.hf = kv(a->h);
+  p.h0f = kv(a->h0);
+  p.da = kv(a->da);
+  p.dh0 = kv(a->dh0);
   p.ws = a->workspace;
   hipError_t e = launch_lscan(p, a->algo, a->dtype, (hipStream_t)stream);
-  if (e != hipSuccess) return hip_fail(e, "ssm_lscan_bwd");
-  LscanGradParams g;
-  memset(&g, 0, sizeof(g));
-  g.B = a->batch;
-  g.L = a->seqlen;
-  g.M = a->width;
-  g.reverse = a->reverse != 0;
-  g.a = kv(a->a);
-  g.h0 = kv(a->h0);
-  g.h = kv(a->h);
-  g.db = kv(a->db);
-  g.da = kv(a->da);
-  g.dh0 = kv(a->dh0);
-  e = launch_lscan_grad(g, a->dtype, (hipStream_t)stream);
   return e == hipSuccess ? ok() : hip_fail(e, "ssm_lscan_bwd");
 }
 

@@ -174,14 +174,10 @@ struct LscanParams {
   int chunk;    // steps per chunk
   int reverse, shift;
   KView a, b, h0, h;  // h0: (B, M) with strides s0, s1
+  // Adjoint (hf set): the scan's values are lambda and go to h (= db); hf is the forward scan's
+  // states and h0f its initial state; da and dh0 are written with lambda.
+  KView hf, h0f, da, dh0;
   void *ws;           // chunked: 3 x (B, nc, M) state type (P, E, h_in)
-};
-
-// da_t = lambda_t h_prev(t) and dh0 = a_first lambda_first; `reverse` is the forward's direction.
-struct LscanGradParams {
-  int64_t B, L, M;
-  int reverse;
-  KView a, h0, h, db, da, dh0;  // db holds lambda
 };
 
 // Materialized discretization on contiguous (B, L, D, N) tensors.
@@ -282,7 +278,6 @@ hipError_t launch_bwd(const BwdParams &p, int dtype, int method, int np, hipStre
 hipError_t launch_bwd_finalize(const FinParams &p, int dtype, hipStream_t s);
 hipError_t launch_step(const StepParams &p, int dtype, int method, int np, hipStream_t s);
 hipError_t launch_lscan(const LscanParams &p, int algo, int dtype, hipStream_t s);
-hipError_t launch_lscan_grad(const LscanGradParams &p, int dtype, hipStream_t s);
 // Channels per workgroup of the discretize backward (its dB partial-sum tile).
 inline int disc_channels(int np) { return kThreads / np; }
 hipError_t launch_conv(const ConvParams &p, int dtype, bool bwd, hipStream_t s);

@@ -1,0 +1,67 @@
+"""GPU: the tiled walk of the linear scans at the edges of its tiles -- lengths around one and two
+tiles (128 steps; 64 for hillis_steele and for the forward walk with 4 row lanes), widths that
+fill no 64-recurrence workgroup, both sides of the chunked algorithm's one-pass rule, the adjoint
+with and without h0, strided views, both directions -- against the recurrence in float64."""
+
+import pytest
+import torch
+
+from parity import close
+from ssm_scan import scan as S
+
+pytestmark = pytest.mark.gpu
+ALGOS = list(S.SCANS)
+
+
+def _ref(a, b, h0, dh, reverse):
+    """h, da, db, dh0 of the recurrence, step by step in float64."""
+    a, b, dh = (t.double().flip(1) if reverse else t.double() for t in (a, b, dh))
+    h = torch.zeros_like(a[:, 0]) if h0 is None else h0.double()
+    hp, hs = [], []
+    for t in range(a.shape[1]):
+        hp.append(h)
+        h = a[:, t] * h + b[:, t]
+        hs.append(h)
+    lam, mu = [], torch.zeros_like(h)
+    for t in reversed(range(a.shape[1])):
+        lam.append(dh[:, t] + mu)
+        mu = a[:, t] * lam[-1]
+    lam = torch.stack(lam[::-1], 1)
+    out = [torch.stack(hs, 1), lam * torch.stack(hp, 1), lam]
+    return [t.flip(1) if reverse else t for t in out] + [mu]
+
+
+# (B, L, M): one workgroup; ragged; 160 workgroups and one fewer; 512 and 1,024 (4 and 8 row lanes)
+SHAPES = [(1, 1, 1), (1, 15, 64), (2, 64, 65), (1, 127, 63), (2, 128, 64), (1, 129, 130), (1, 257, 70),
+          (1, 63, 10240), (1, 130, 10177), (1, 66, 10176), (2, 70, 16384), (4, 33, 16384)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("algo", ALGOS)
+def test_walk_edges(algo, shape):
+    B, L, M = shape
+    g = torch.Generator(device="cuda").manual_seed(L * 7 + M)
+    a = torch.rand(B, L, M, generator=g, device="cuda") * 0.5 + 0.5
+    b, dh = (torch.randn(B, L, M, generator=g, device="cuda") for _ in range(2))
+    for h0, reverse in ((torch.randn(B, M, generator=g, device="cuda"), False), (None, True)):
+        leaves = [t.detach().requires_grad_() for t in (a, b) + ((h0,) if h0 is not None else ())]
+        h = S._scan(algo, *leaves, reverse=reverse)
+        grads = torch.autograd.grad(h, leaves, dh)
+        refs = _ref(a, b, h0, dh, reverse)
+        # da = lambda h_prev: each factor within a few ulps of its largest magnitude, times the other
+        da_atol = max(1e-5, 16 * 2.0 ** -24 * refs[0].abs().max().item() * refs[2].abs().max().item())
+        for name, got, ref in zip(("h", "da", "db", "dh0"), (h.detach(), *grads), refs):
+            close(got, ref, name=name, **({"atol": da_atol} if name == "da" else {}))
+
+
+@pytest.mark.parametrize("algo", ALGOS)
+def test_walk_strided_and_float64(algo):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    B, L, M = 2, 131, 37
+    a = (torch.rand(B, M, L, generator=g, device="cuda", dtype=torch.float64) * 0.5 + 0.5).transpose(1, 2)
+    b, dh = (torch.randn(B, L, 2 * M, generator=g, device="cuda", dtype=torch.float64)[..., ::2] for _ in range(2))
+    leaves = [t.detach().requires_grad_() for t in (a, b)]
+    h = S._scan(algo, *leaves)
+    grads = torch.autograd.grad(h, leaves, dh)
+    for got, ref in zip((h.detach(), *grads), _ref(a, b, None, dh, False)):
+        torch.testing.assert_close(got, ref, rtol=1e-12, atol=1e-12)
