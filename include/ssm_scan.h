@@ -286,6 +286,37 @@ typedef struct ssm_lscan_bwd_args {
   int64_t workspace_bytes;
 } ssm_lscan_bwd_args;
 
+/* ------------------------------------------------------------------ composed selective scan
+ * SelectiveScanFn with a named algorithm (models/scan.py:193-255): discretize, scan, contract with
+ * C, and its backward by recompute and an adjoint scan -- in one kernel per direction that keeps a,
+ * b, h and their gradients in registers tile by tile in time.  Every tensor is float32 or float64
+ * (dtype) with any strides; 64 steps of a batch row of x, delta, dy, Bm and Cm span less than 2^31
+ * bytes.  The forward
+ * writes the state entering every time tile of ssm_cscan_tile() steps to `saved` when given:
+ * (B, ceil(L / tile), D, N), strides (b, tile, d), states consecutive; the backward reads it. */
+typedef struct ssm_cscan_args {
+  int64_t batch, seqlen, dim, dstate;
+  int32_t algo;            /* SSM_SCAN_SEQUENTIAL .. SSM_SCAN_CHUNKED */
+  int32_t method;          /* SSM_ZOH / SSM_EULER / SSM_BILINEAR */
+  int32_t dtype;           /* SSM_F32 or SSM_F64 */
+  int32_t reserved0;
+  ssm_tensor x, delta;     /* (B,L,D) */
+  ssm_tensor A;            /* (D,N) */
+  ssm_tensor Bm, Cm;       /* (B,L,N) */
+  ssm_tensor h0;           /* (B,D,N) optional */
+  ssm_tensor y;            /* forward: (B,L,D) */
+  ssm_tensor last;         /* forward: (B,D,N) optional */
+  ssm_tensor saved;        /* forward: optional; backward: required */
+  ssm_tensor dy;           /* backward: (B,L,D) */
+  ssm_tensor dlast;        /* backward: (B,D,N) optional */
+  ssm_tensor dx, ddelta;   /* backward: (B,L,D) */
+  ssm_tensor dA;           /* backward: (D,N) */
+  ssm_tensor dBm, dCm;     /* backward: (B,L,N) */
+  ssm_tensor dh0;          /* backward: (B,D,N) optional */
+  void *workspace;         /* backward: ssm_cscan_workspace_bytes() */
+  int64_t workspace_bytes;
+} ssm_cscan_args;
+
 /* ------------------------------------------------------------------ discretization
  * models/scan.py:39-55, materialized: a, b (B,L,D,N), contiguous.  The backward maps
  * (da, db) to (ddelta, dA, dBm, dx) exactly as autograd does through discretize
@@ -358,6 +389,7 @@ int ssm_decode_check(const ssm_decode_args *args);
 int ssm_decode_stack_check(const ssm_decode_stack_args *args);
 int ssm_lscan_check(const ssm_lscan_args *args);
 int ssm_lscan_bwd_check(const ssm_lscan_bwd_args *args);
+int ssm_cscan_check(const ssm_cscan_args *args);
 int ssm_disc_check(const ssm_disc_args *args);
 int ssm_conv_check(const ssm_conv_args *args);
 int ssm_norm_check(const ssm_norm_args *args);
@@ -368,6 +400,7 @@ int64_t ssm_fwd_workspace_bytes(const ssm_fwd_args *args);
 int64_t ssm_bwd_workspace_bytes(const ssm_bwd_args *args);
 int64_t ssm_lscan_workspace_bytes(const ssm_lscan_args *args);
 int64_t ssm_lscan_bwd_workspace_bytes(const ssm_lscan_bwd_args *args);
+int64_t ssm_cscan_workspace_bytes(const ssm_cscan_args *args);
 int64_t ssm_disc_workspace_bytes(const ssm_disc_args *args);
 int64_t ssm_conv_workspace_bytes(const ssm_conv_args *args);
 int64_t ssm_norm_workspace_bytes(const ssm_norm_args *args);
@@ -388,6 +421,8 @@ int ssm_decode_step(const ssm_decode_args *args, void *stream);
 int ssm_decode_stack(const ssm_decode_stack_args *args, void *stream);
 int ssm_lscan(const ssm_lscan_args *args, void *stream);
 int ssm_lscan_bwd(const ssm_lscan_bwd_args *args, void *stream);
+int ssm_cscan_fwd(const ssm_cscan_args *args, void *stream);
+int ssm_cscan_bwd(const ssm_cscan_args *args, void *stream);
 int ssm_disc_fwd(const ssm_disc_args *args, void *stream);
 int ssm_disc_bwd(const ssm_disc_args *args, void *stream);
 int ssm_conv_fwd(const ssm_conv_args *args, void *stream);
@@ -410,6 +445,7 @@ int ssm_fwd_noalloc(const ssm_fwd_args *args, void *stream);
 /* ------------------------------------------------------------------ plans (host-only, exact integers)
  * The reference's integer planning functions, returned bit-exactly. */
 int64_t ssm_default_chunk(int64_t seqlen);                        /* models/scan.py:138-139 */
+int64_t ssm_cscan_tile(int32_t algo, int32_t dtype);  /* steps per time tile of ssm_cscan; no counterpart */
 int64_t ssm_scan_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate,
                         int64_t d_block, int64_t *bounds, int64_t capacity);
                                                                   /* models/scan.py:185-190; writes

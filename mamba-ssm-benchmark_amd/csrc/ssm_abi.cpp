@@ -725,6 +725,92 @@ int ssm_disc_bwd(const ssm_disc_args *a, void *stream) {
   return e == hipSuccess ? ok() : hip_fail(e, "ssm_disc_bwd");
 }
 
+// ------------------------------------------------------------------ composed selective scan
+int64_t ssm_cscan_tile(int32_t algo, int32_t dtype) {
+  if (algo < SSM_SCAN_SEQUENTIAL || algo > SSM_SCAN_CHUNKED || (dtype != SSM_F32 && dtype != SSM_F64)) return -1;
+  return csc_tile(algo, dtype == SSM_F64);
+}
+
+// The composed kernels address a time tile (up to 64 steps) by 31-bit byte offsets.
+static int csc_offsets(const ssm_tensor &t, int64_t extent, int esize, const char *name) {
+  const int64_t s1 = t.stride[1], s2 = t.stride[2], lim = 1LL << 31;
+  if (s1 < 0 || s2 < 0 || s1 >= lim || s2 >= lim || (s2 * (extent - 1) + 63 * s1 + 1) * esize >= lim)
+    return fail(SSM_EINVAL, "%s: strides (%lld, %lld) too large for extent %lld", name, (long long)s1, (long long)s2,
+                (long long)extent);
+  return 0;
+}
+
+int ssm_cscan_check(const ssm_cscan_args *a) {
+  if (!a) return fail(SSM_EINVAL, "null args");
+  int rc = check_common(a->batch, a->seqlen, a->dim, a->dstate, a->method, a->dtype);
+  if (rc) return rc;
+  if (a->algo < SSM_SCAN_SEQUENTIAL || a->algo > SSM_SCAN_CHUNKED)
+    return fail(SSM_EINVAL, "unknown scan algorithm %d (sequential=1 .. chunked=4)", a->algo);
+  if (a->dtype != SSM_F32 && a->dtype != SSM_F64) return fail(SSM_EINVAL, "composed scans take float32 or float64");
+  REQUIRE(a->x, "x");
+  REQUIRE(a->delta, "delta");
+  REQUIRE(a->A, "A");
+  REQUIRE(a->Bm, "Bm");
+  REQUIRE(a->Cm, "Cm");
+  const int es = state_size(a->dtype);
+  if ((rc = csc_offsets(a->x, a->dim, es, "x")) || (rc = csc_offsets(a->delta, a->dim, es, "delta")) ||
+      (rc = csc_offsets(a->Bm, a->dstate, es, "Bm")) || (rc = csc_offsets(a->Cm, a->dstate, es, "Cm")))
+    return rc;
+  return ok();
+}
+
+static CscParams csc_params(const ssm_cscan_args *a) {
+  CscParams p;
+  memset(&p, 0, sizeof(p));
+  p.B = a->batch; p.L = a->seqlen; p.D = a->dim; p.N = a->dstate;
+  p.ntiles = cdiv(a->dim, 64 / padded_n(a->dstate));
+  p.x = kv(a->x); p.dt = kv(a->delta); p.A = kv(a->A); p.Bm = kv(a->Bm); p.Cm = kv(a->Cm); p.h0 = kv(a->h0);
+  p.y = kv(a->y); p.last = kv(a->last); p.saved = kv(a->saved);
+  p.dy = kv(a->dy); p.dlast = kv(a->dlast); p.dx = kv(a->dx); p.ddelta = kv(a->ddelta);
+  p.dA = kv(a->dA); p.dB = kv(a->dBm); p.dC = kv(a->dCm); p.dh0 = kv(a->dh0);
+  return p;
+}
+
+static int64_t csc_ws_bc(const ssm_cscan_args *a, const CscParams &p) {
+  return align256(a->batch * p.ntiles * a->seqlen * 2 * padded_n(a->dstate) * state_size(a->dtype));
+}
+
+int64_t ssm_cscan_workspace_bytes(const ssm_cscan_args *a) {
+  if (ssm_cscan_check(a)) return -1;
+  return csc_ws_bc(a, csc_params(a)) + align256(a->batch * a->dim * a->dstate * 8);
+}
+
+int ssm_cscan_fwd(const ssm_cscan_args *a, void *stream) {
+  int rc = ssm_cscan_check(a);
+  if (rc) return rc;
+  REQUIRE(a->y, "y");
+  const hipError_t e = launch_csc(csc_params(a), a->algo, a->dtype, a->method, padded_n(a->dstate), false,
+                                  (hipStream_t)stream);
+  return e == hipSuccess ? ok() : hip_fail(e, "ssm_cscan_fwd");
+}
+
+int ssm_cscan_bwd(const ssm_cscan_args *a, void *stream) {
+  int rc = ssm_cscan_check(a);
+  if (rc) return rc;
+  REQUIRE(a->saved, "saved");
+  REQUIRE(a->dy, "dy");
+  REQUIRE(a->dx, "dx");
+  REQUIRE(a->ddelta, "ddelta");
+  REQUIRE(a->dA, "dA");
+  REQUIRE(a->dBm, "dBm");
+  REQUIRE(a->dCm, "dCm");
+  if (has(a->dh0) && !has(a->h0)) return fail(SSM_EINVAL, "dh0 given without h0");
+  if ((rc = csc_offsets(a->dy, a->dim, state_size(a->dtype), "dy"))) return rc;
+  CscParams p = csc_params(a);
+  const int64_t bc = csc_ws_bc(a, p), need = bc + align256(a->batch * a->dim * a->dstate * 8);
+  if (!a->workspace || a->workspace_bytes < need)
+    return fail(SSM_ESPACE, "workspace of %lld bytes required", (long long)need);
+  p.ws_bc = a->workspace;
+  p.ws_dA = (char *)a->workspace + bc;
+  const hipError_t e = launch_csc(p, a->algo, a->dtype, a->method, padded_n(a->dstate), true, (hipStream_t)stream);
+  return e == hipSuccess ? ok() : hip_fail(e, "ssm_cscan_bwd");
+}
+
 // ------------------------------------------------------------------ fused decode layer
 int ssm_decode_check(const ssm_decode_args *a) {
   if (!a) return fail(SSM_EINVAL, "null args");

@@ -191,6 +191,22 @@ struct DiscParams {
   void *ws_dA;  // (ngroups, D, N) partial sums over each group of rows (float64 running sums)
 };
 
+// The composed selective scan (discretize, scan by a named algorithm, contract) without
+// materialized (B, L, D, N) tensors.  A time tile is 8 row lanes (wavefronts) x 8 steps; 4 x 4 for
+// float64 Hillis-Steele, whose LDS holds every step of a tile four times.
+__host__ __device__ constexpr int csc_row_lanes(int algo, bool f64) { return algo == 2 && f64 ? 4 : 8; }
+__host__ __device__ constexpr int csc_tile(int algo, bool f64) { return algo == 2 && f64 ? 16 : 64; }
+struct CscParams {
+  int64_t B, L, D, N;
+  int64_t ntiles;  // channel tiles of the dB / dC partials
+  KView x, dt, A, Bm, Cm, h0, y, last;
+  KView saved;     // state entering each time tile: strides (b, tile, d), states consecutive
+  KView dy, dlast, dx, ddelta, dA, dB, dC, dh0;
+  void *ws_bc;     // (B, ntiles, L, 2, NP) state type: dB and dC partials over a tile's channels
+  void *ws_dA;     // (B, D, N) float64
+};
+hipError_t launch_csc(const CscParams &p, int algo, int dtype, int method, int np, bool bwd, hipStream_t s);
+
 // Causal depthwise conv over (B, L, D) views; a lane owns (b, d, one block of TB steps).
 // Causal conv: a workgroup covers kConvDG channels x kConvTG lanes of kConvTT time steps
 // (kConvTT >= W - 1 for every width <= 8).

@@ -40,6 +40,7 @@
 #include "ssm_dpp.hpp"
 #include "ssm_internal.hpp"
 #include "ssm_tiles.hpp"
+#include "ssm_tilescan.hpp"
 #include "ssm_wave.hpp"
 
 namespace ssm {
@@ -88,38 +89,21 @@ struct Chain {
 };
 
 // ------------------------------------------------------------------ the tiled walk
-enum { kSeq = 1, kHs = 2, kBl = 3, kChunk = 4 };  // algorithm ids of the C ABI
 constexpr int kScanMC = 64;   // recurrences per workgroup
 // Steps per row lane and tile (Hillis-Steele keeps every step of a tile in LDS twice).
 constexpr int scan_rows(int algo) { return algo == kHs ? 8 : 16; }
-
-// What the row lanes exchange through LDS.
-template <typename CT, int ALGO, int RL> struct WalkLds {  // sequential: the state handed over
-  CT h[kScanMC];
-};
-template <typename CT, int RL> struct WalkLds<CT, kHs, RL> {
-  static constexpr int T = RL * scan_rows(kHs);
-  CT A[2][T][kScanMC], S[2][T][kScanMC], last[kScanMC];
-};
-template <typename CT, int RL> struct WalkLds<CT, kBl, RL> {
-  CT A[RL][kScanMC], S[RL][kScanMC], last[kScanMC];
-};
-template <typename CT, int RL> struct WalkLds<CT, kChunk, RL> {
-  CT P[2][RL][kScanMC], E[2][RL][kScanMC];
-};
 
 template <typename CT, int ALGO, int RL, bool GRAD>
 __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P) {
   constexpr int R = scan_rows(ALGO), T = RL * R;
   static_assert(kScanMC == kWave, "a row lane is a wavefront");
-  __shared__ WalkLds<CT, ALGO, RL> X;
+  __shared__ TileLds<CT, ALGO, RL, R> X;
   const int mi = threadIdx.x % kScanMC, tr = __builtin_amdgcn_readfirstlane(threadIdx.x / kScanMC);
   const int64_t m = (int64_t)blockIdx.x * kScanMC + mi;
   const bool mval = m < P.M;
   Chain<CT> ch{P, (int64_t)blockIdx.y, mval ? m : P.M - 1};
   const int L = (int)P.L;
-  // the row lane's r-th step of a tile: 16 consecutive steps, or every RL-th (Hillis-Steele)
-  auto step = [&](int r) { return ALGO == kHs ? tr + RL * r : tr * R + r; };
+  auto step = [&](int r) { return tile_step<ALGO, RL, R>(tr, r); };
   CT carry = ch.h0();
   CT na[R], nb[R], nh[GRAD ? R : 1];
   auto fetch = [&](int base) {  // reads at clamped positions
@@ -143,165 +127,12 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
       if constexpr (GRAD) hp[r] = nh[r];
     }
     if (base + T < L) fetch(base + T);
-    auto put = [&](int r, CT v) {
+    CT hin;
+    tile_scan<CT, ALGO, RL, R>(X, a, b, carry, hin, tr, mi, buf);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
       const int pos = base + step(r);
-      if (mval && pos < L) ch.template put<GRAD>(pos, v, hp[GRAD ? r : 0]);
-    };
-    if constexpr (ALGO == kSeq) {
-      // a turn is a handover and 16 dependent updates; the stores follow outside it
-#pragma unroll
-      for (int q = 0; q < RL; ++q) {
-        if (q == tr) {
-          CT h = base == 0 && q == 0 ? carry : X.h[mi];
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            h = fma(a[r], h, b[r]);
-            b[r] = h;
-          }
-          X.h[mi] = h;
-        }
-        lds_barrier();
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) put(r, b[r]);
-    } else if constexpr (ALGO == kHs) {
-      // At offset o every step k >= o composes with step k - o of the previous pass.  The
-      // offsets below RL pair different row lanes (step k - o is in row lane tr - o, or one
-      // register lower in row lane tr - o + RL), the others registers of one lane.
-      if (tr == 0) b[0] = fma(a[0], carry, b[0]);  // fold the incoming state into the first element
-#pragma unroll
-      for (int o = 1; o < RL; o *= 2) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          X.A[buf][step(r)][mi] = a[r];
-          X.S[buf][step(r)][mi] = b[r];
-        }
-        lds_barrier();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int k = step(r);
-          if (k >= o) {
-            b[r] = fma(a[r], X.S[buf][k - o][mi], b[r]);
-            a[r] = a[r] * X.A[buf][k - o][mi];
-          }
-        }
-        buf ^= 1;  // the next pass (or tile) writes beside the steps still being read
-      }
-#pragma unroll
-      for (int j = 1; j < R; j *= 2) {  // descending r reads the previous pass's r - j
-#pragma unroll
-        for (int r = R - 1; r >= j; --r) {
-          b[r] = fma(a[r], b[r - j], b[r]);
-          a[r] = a[r] * a[r - j];
-        }
-      }
-      if (tr == RL - 1) X.last[mi] = b[R - 1];  // step T - 1: the state entering the next tile
-      lds_barrier();
-      carry = X.last[mi];
-#pragma unroll
-      for (int r = 0; r < R; ++r) put(r, b[r]);
-    } else if constexpr (ALGO == kBl) {
-      // Tree levels of span 2..R are register operations of one lane; the levels above combine
-      // the block roots, which every lane of a column reads from LDS and sweeps itself (the
-      // same combines in every lane, so the same bits).
-      CT A[R], S[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        A[r] = a[r];
-        S[r] = b[r];
-      }
-#pragma unroll
-      for (int sp = 2; sp <= R; sp *= 2) {  // up-sweep: right <- right o left at nodes (j + 1) sp - 1
-#pragma unroll
-        for (int k = sp - 1; k < R; k += sp) {
-          const int l = k - sp / 2;
-          S[k] = fma(A[k], S[l], S[k]);
-          A[k] = A[k] * A[l];
-        }
-      }
-      X.A[tr][mi] = A[R - 1];
-      X.S[tr][mi] = S[R - 1];
-      lds_barrier();
-      CT rA[RL], rS[RL];
-#pragma unroll
-      for (int q = 0; q < RL; ++q) {
-        rA[q] = X.A[q][mi];
-        rS[q] = X.S[q][mi];
-      }
-#pragma unroll
-      for (int sp = 2; sp <= RL; sp *= 2) {
-#pragma unroll
-        for (int k = sp - 1; k < RL; k += sp) {
-          const int l = k - sp / 2;
-          rS[k] = fma(rA[k], rS[l], rS[k]);
-          rA[k] = rA[k] * rA[l];
-        }
-      }
-      // the root set to the identity, then the down-sweep (left <- right; right <- left_old o
-      // right): each root becomes the composition of the blocks before it
-      rA[RL - 1] = 1;
-      rS[RL - 1] = 0;
-#pragma unroll
-      for (int sp = RL; sp >= 2; sp /= 2) {
-#pragma unroll
-        for (int k = sp - 1; k < RL; k += sp) {
-          const int l = k - sp / 2;
-          const CT tA = rA[l], tS = rS[l];
-          rA[l] = rA[k];
-          rS[l] = rS[k];
-          rS[k] = fma(rS[k], tA, tS);
-          rA[k] = rA[k] * tA;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < RL; ++q) {  // this row lane's root
-        if (q == tr) {
-          A[R - 1] = rA[q];
-          S[R - 1] = rS[q];
-        }
-      }
-#pragma unroll
-      for (int sp = R; sp >= 2; sp /= 2) {
-#pragma unroll
-        for (int k = sp - 1; k < R; k += sp) {
-          const int l = k - sp / 2;
-          const CT tA = A[l], tS = S[l];
-          A[l] = A[k];
-          S[l] = S[k];
-          S[k] = fma(S[k], tA, tS);
-          A[k] = A[k] * tA;
-        }
-      }
-      // exclusive prefixes: the state entering step k is A_k h_in + S_k
-#pragma unroll
-      for (int r = 0; r < R; ++r) b[r] = fma(a[r], fma(A[r], carry, S[r]), b[r]);
-      if (tr == RL - 1) X.last[mi] = b[R - 1];  // step T - 1: the state entering the next tile
-      lds_barrier();
-      carry = X.last[mi];
-#pragma unroll
-      for (int r = 0; r < R; ++r) put(r, b[r]);
-    } else {
-      CT pr = a[0], e = b[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        e = fma(a[r], e, b[r]);
-        pr *= a[r];
-      }
-      X.P[buf][tr][mi] = pr;
-      X.E[buf][tr][mi] = e;
-      lds_barrier();
-      CT h = carry;
-#pragma unroll
-      for (int q = 0; q < RL; ++q) {  // the same folds in every lane, so the same bits
-        if (q == tr) h = carry;       // the state entering this row lane's chunk
-        carry = fma(X.P[buf][q][mi], carry, X.E[buf][q][mi]);
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        h = fma(a[r], h, b[r]);
-        put(r, h);
-      }
-      buf ^= 1;  // the next tile's summaries go beside the ones still being read
+      if (mval && pos < L) ch.template put<GRAD>(pos, b[r], hp[GRAD ? r : 0]);
     }
   }
 }

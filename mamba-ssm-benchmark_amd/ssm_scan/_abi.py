@@ -105,6 +105,16 @@ class LscanBwdArgs(ctypes.Structure):
                 ("workspace", c_vp), ("workspace_bytes", c_i64)]
 
 
+class CscanArgs(ctypes.Structure):
+    _fields_ = [("batch", c_i64), ("seqlen", c_i64), ("dim", c_i64), ("dstate", c_i64),
+                ("algo", c_i32), ("method", c_i32), ("dtype", c_i32), ("reserved0", c_i32),
+                ("x", Tensor), ("delta", Tensor), ("A", Tensor), ("Bm", Tensor), ("Cm", Tensor),
+                ("h0", Tensor), ("y", Tensor), ("last", Tensor), ("saved", Tensor),
+                ("dy", Tensor), ("dlast", Tensor), ("dx", Tensor), ("ddelta", Tensor), ("dA", Tensor),
+                ("dBm", Tensor), ("dCm", Tensor), ("dh0", Tensor),
+                ("workspace", c_vp), ("workspace_bytes", c_i64)]
+
+
 class DiscArgs(ctypes.Structure):
     _fields_ = [("batch", c_i64), ("seqlen", c_i64), ("dim", c_i64), ("dstate", c_i64),
                 ("method", c_i32), ("dtype", c_i32),
@@ -142,6 +152,7 @@ _SIGS = {
     "ssm_decode_stack_check": (c_i32, [ctypes.POINTER(DecodeStackArgs)]),
     "ssm_lscan_check": (c_i32, [ctypes.POINTER(LscanArgs)]),
     "ssm_lscan_bwd_check": (c_i32, [ctypes.POINTER(LscanBwdArgs)]),
+    "ssm_cscan_check": (c_i32, [ctypes.POINTER(CscanArgs)]),
     "ssm_disc_check": (c_i32, [ctypes.POINTER(DiscArgs)]),
     "ssm_conv_check": (c_i32, [ctypes.POINTER(ConvArgs)]),
     "ssm_norm_check": (c_i32, [ctypes.POINTER(NormArgs)]),
@@ -150,6 +161,7 @@ _SIGS = {
     "ssm_bwd_workspace_bytes": (c_i64, [ctypes.POINTER(BwdArgs)]),
     "ssm_lscan_workspace_bytes": (c_i64, [ctypes.POINTER(LscanArgs)]),
     "ssm_lscan_bwd_workspace_bytes": (c_i64, [ctypes.POINTER(LscanBwdArgs)]),
+    "ssm_cscan_workspace_bytes": (c_i64, [ctypes.POINTER(CscanArgs)]),
     "ssm_disc_workspace_bytes": (c_i64, [ctypes.POINTER(DiscArgs)]),
     "ssm_conv_workspace_bytes": (c_i64, [ctypes.POINTER(ConvArgs)]),
     "ssm_norm_workspace_bytes": (c_i64, [ctypes.POINTER(NormArgs)]),
@@ -163,12 +175,15 @@ _SIGS = {
     "ssm_decode_stack": (c_i32, [ctypes.POINTER(DecodeStackArgs), c_vp]),
     "ssm_lscan": (c_i32, [ctypes.POINTER(LscanArgs), c_vp]),
     "ssm_lscan_bwd": (c_i32, [ctypes.POINTER(LscanBwdArgs), c_vp]),
+    "ssm_cscan_fwd": (c_i32, [ctypes.POINTER(CscanArgs), c_vp]),
+    "ssm_cscan_bwd": (c_i32, [ctypes.POINTER(CscanArgs), c_vp]),
     "ssm_disc_fwd": (c_i32, [ctypes.POINTER(DiscArgs), c_vp]),
     "ssm_disc_bwd": (c_i32, [ctypes.POINTER(DiscArgs), c_vp]),
     "ssm_conv_fwd": (c_i32, [ctypes.POINTER(ConvArgs), c_vp]),
     "ssm_conv_bwd": (c_i32, [ctypes.POINTER(ConvArgs), c_vp]),
     "ssm_norm_fwd": (c_i32, [ctypes.POINTER(NormArgs), c_vp]),
     "ssm_norm_bwd": (c_i32, [ctypes.POINTER(NormArgs), c_vp]),
+    "ssm_cscan_tile": (c_i64, [c_i32, c_i32]),
     "ssm_default_chunk": (c_i64, [c_i64]),
     "ssm_scan_blocks": (c_i64, [c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.POINTER(c_i64), c_i64]),
     "ssm_block_d": (c_i64, [c_i64, c_i64]),

@@ -10,8 +10,8 @@ as models/mamba.py:120-121 switch by changing the import:
   scan_blelloch     models/scan.py:101-135    | differentiable through ssm_lscan_bwd
   scan_chunked      models/scan.py:142-165   /
   SCANS, default_chunk, SCAN_ELEMENT_BUDGET, _blocks   models/scan.py:138-190
-  SelectiveScanFn   models/scan.py:193-255   per channel tile: discretize -> scan -> contract,
-                                             backward by recompute + reverse scan
+  SelectiveScanFn   models/scan.py:193-255   discretize -> scan -> contract in one kernel per
+                                             direction, backward by recompute + reverse scan
   selective_scan_reference  models/scan.py:264-274   the time loop; runs on the fused engine,
                                              which walks the same recurrence step by step
   selective_scan    models/scan.py:277-299   dispatcher ('triton' and 'auto' select the fused
@@ -242,114 +242,112 @@ def _scan_algo(name):
 
 
 # ------------------------------------------------------------------ composed selective scan
-def _scan_into(algo, chunk, a, b, h0):
-    """Forward scan of (B, L, d, N) tensors into a new (B, L, d, N) h."""
-    Bsz, L, d, N = a.shape
-    h = torch.empty_like(a)
-    args = _abi.LscanArgs()
-    _lscan_common(args, a.view(Bsz, L, d * N), algo, chunk, False)
-    args.a = _abi.view(a.view(Bsz, L, d * N))
-    args.b = _abi.view(b.view(Bsz, L, d * N))
-    args.h0 = _abi.view(None if h0 is None else h0.reshape(Bsz, d * N))
-    args.h = _abi.view(h.view(Bsz, L, d * N))
-    lib = _abi.lib()
-    nbytes = lib.ssm_lscan_workspace_bytes(ctypes.byref(args))
-    if nbytes < 0:
-        _abi.check(lib.ssm_lscan_check(ctypes.byref(args)), "ssm_lscan")
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=a.device) if nbytes else None
-    if ws is not None:
-        args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-    _launch("ssm_lscan", lib.ssm_lscan, args, a.device)
-    return h
+_CSCAN_WORKSPACE = 1 << 28   # bytes of dB / dC partials per backward launch
 
 
-def _disc_fwd(delta, A, Bm, x, method):
-    Bsz, L, d = x.shape
-    N = A.shape[1]
-    a = torch.empty((Bsz, L, d, N), dtype=delta.dtype, device=x.device)
-    b = torch.empty_like(a)
-    args = _disc_args(delta, A, Bm, x, method)
-    args.a, args.b = a.data_ptr(), b.data_ptr()
-    _launch("ssm_disc_fwd", _abi.lib().ssm_disc_fwd, args, x.device)
-    return a, b
+def _cscan_args(x, delta, A, Bm, Cm, h0, saved, i, j, method, algo):
+    """The operands both directions share; x and delta are channels i..j already, the rest whole."""
+    args = _abi.CscanArgs()
+    args.batch, args.seqlen, args.dim, args.dstate = *x.shape, A.shape[1]
+    args.algo, args.method, args.dtype = algo, METHODS[method], _abi.DTYPE_CODE[x.dtype]
+    args.x, args.delta, args.A = _abi.view(x), _abi.view(delta), _abi.view(A[i:j])
+    args.Bm, args.Cm = _abi.view(Bm), _abi.view(Cm)
+    args.h0 = _abi.view(None if h0 is None else h0[:, i:j])
+    if saved is not None:
+        args.saved = _abi.Tensor(saved[:, :, i:j].data_ptr(), saved.stride()[:3])
+    return args
+
+
+def _cscan_channels(x, N, d_block, workspace):
+    """Channel tiles of the launches: those of d_block, else all channels at once up to 2^21 and,
+    with `workspace`, as many as keep the backward's partials (2 x L x NP per 64 / NP channels and
+    batch row) within _CSCAN_WORKSPACE."""
+    Bsz, L, D = x.shape
+    step = 1 << 21
+    if d_block and d_block > 0:
+        step = min(step, d_block)
+    elif workspace and N <= 64:
+        NP = max(8, 1 << (N - 1).bit_length())
+        step = min(step, max(1, _CSCAN_WORKSPACE // (Bsz * L * 2 * NP * x.element_size())) * (64 // NP))
+    return [(i, min(D, i + step)) for i in range(0, D, step)]
+
+
+def _steps_fit(t):
+    """t, or a contiguous copy where 64 steps of a batch row span 2 GiB (the kernels' offsets)."""
+    fits = (t.stride(2) * (t.shape[2] - 1) + 63 * t.stride(1) + 1) * t.element_size() < 1 << 31
+    return t if fits else t.contiguous()
 
 
 class SelectiveScanFn(torch.autograd.Function):
-    """y, last = selective scan with recomputation (models/scan.py:193-255).
+    """y, last = selective scan by a named algorithm (models/scan.py:193-255).
 
-    Saves only x, delta, A, Bm, Cm, h0.  Channels run in tiles of d_block (default sized to
-    SCAN_ELEMENT_BUDGET); per tile the forward discretizes into (B, L, d, N), scans with the
-    chosen algorithm and contracts with C; the backward recomputes the states, runs the
-    adjoint scan lambda_t = g_t + a_{t+1} lambda_{t+1} with the same algorithm and maps
-    (da, db) = (lambda h_{t-1}, lambda) back through the discretization."""
+    One kernel discretizes, scans and contracts with C tile by tile in time (ssm_cscan), so no
+    (B, L, D, N) tensor exists; saved for the backward are x, delta, A, Bm, Cm, h0 and the state
+    entering every time tile.  The backward recomputes the states tile by tile, runs the adjoint
+    scan lambda_t = g_t + a_{t+1} lambda_{t+1} with the same algorithm and maps (da, db) =
+    (lambda h_{t-1}, lambda) back through the discretization, in channel tiles of d_block
+    (default: _CSCAN_WORKSPACE).  chunk_size is the chunk of the linear scan over materialized
+    tensors; here a chunk is a wavefront's part of a time tile."""
 
     @staticmethod
     def forward(ctx, x, delta, A, Bm, Cm, h0, method, scan_name, d_block, chunk_size):
         algo = _scan_algo(scan_name)
         if method not in DISCRETIZATIONS:
             raise ValueError(f"unknown discretization {method!r}")
+        chunk = int(chunk_size or 0)
+        if not 0 <= chunk < 1 << 30:
+            raise ValueError(f"chunk={chunk} out of range")
         Bsz, L, D = x.shape
         N = A.shape[1]
+        Bm, Cm = _steps_fit(Bm), _steps_fit(Cm)
         y = torch.empty_like(x)
         last = torch.empty(Bsz, D, N, dtype=x.dtype, device=x.device)
-        Cc = Cm.unsqueeze(-1)
-        for i, j in _blocks(x.shape, N, d_block):
-            a, b = _disc_fwd(delta[..., i:j], A[i:j], Bm, x[..., i:j], method)
-            h = _scan_into(algo, chunk_size, a, b, None if h0 is None else h0[:, i:j])
-            del a, b
-            y[..., i:j] = torch.matmul(h, Cc).squeeze(-1)
-            last[:, i:j] = h[:, -1]
-            del h
-        ctx.save_for_backward(x, delta, A, Bm, Cm, h0)
-        ctx.cfg = (method, algo, d_block, chunk_size)
+        lib = _abi.lib()
+        saved = None
+        if any(ctx.needs_input_grad[:6]):
+            tile = lib.ssm_cscan_tile(algo, _abi.DTYPE_CODE[x.dtype])
+            saved = torch.empty(Bsz, -(-L // tile), D, N, dtype=x.dtype, device=x.device)
+        for i, j in _cscan_channels(x, N, None, False):
+            xb, db = _steps_fit(x[..., i:j]), _steps_fit(delta[..., i:j])
+            args = _cscan_args(xb, db, A, Bm, Cm, h0, saved, i, j, method, algo)
+            args.y, args.last = _abi.view(y[..., i:j]), _abi.view(last[:, i:j])
+            _launch("ssm_cscan_fwd", lib.ssm_cscan_fwd, args, x.device)
+        ctx.save_for_backward(x, delta, A, Bm, Cm, h0, saved)
+        ctx.set_materialize_grads(False)   # an unused output passes None (no zero fill)
+        ctx.cfg = (method, algo, d_block)
         return y, last
 
     @staticmethod
     def backward(ctx, dy, dlast):
-        x, delta, A, Bm, Cm, h0 = ctx.saved_tensors
-        method, algo, d_block, chunk_size = ctx.cfg
-        Bsz, L, D = x.shape
+        x, delta, A, Bm, Cm, h0, saved = ctx.saved_tensors
+        method, algo, d_block = ctx.cfg
         N = A.shape[1]
-        dev = x.device
         if dy is None:
             dy = torch.zeros_like(x)
         dx, ddelta, dA = torch.empty_like(x), torch.empty_like(delta), torch.empty_like(A)
-        dBm, dCm = torch.zeros_like(Bm), torch.zeros_like(Cm)
+        dBm = dCm = None
         dh0 = None if h0 is None else torch.empty_like(h0)
         lib = _abi.lib()
-        for i, j in _blocks(x.shape, N, d_block):
-            d = j - i
-            h0_blk = None if h0 is None else h0[:, i:j]
-            a, b = _disc_fwd(delta[..., i:j], A[i:j], Bm, x[..., i:j], method)
-            h = _scan_into(algo, chunk_size, a, b, h0_blk)                 # recompute
-            del b
-            dy_blk = dy[..., i:j]
-            dCm += torch.matmul(dy_blk.unsqueeze(2), h).squeeze(2)
-            g = dy_blk.unsqueeze(-1) * Cm.unsqueeze(2)                       # dL/dh_t (direct)
-            if dlast is not None:
-                g[:, -1] += dlast[:, i:j]
-            da, lam = torch.empty_like(h), torch.empty_like(h)
-            dh0_blk = None if h0 is None else torch.empty((Bsz, d, N), dtype=h.dtype, device=dev)
-            M = d * N
-            lscan_bwd(a.view(Bsz, L, M), None if h0_blk is None else h0_blk.reshape(Bsz, M),
-                      h.view(Bsz, L, M), g.view(Bsz, L, M), da.view(Bsz, L, M), lam.view(Bsz, L, M),
-                      None if dh0_blk is None else dh0_blk.view(Bsz, M), algo, chunk_size, False)
-            del g, h, a
-            if dh0 is not None:
-                dh0[:, i:j] = dh0_blk
-            gB = torch.empty_like(Bm)
-            args = _disc_args(delta[..., i:j], A[i:j], Bm, x[..., i:j], method)
-            args.da, args.db = da.data_ptr(), lam.data_ptr()
-            args.ddelta, args.dx = _abi.view(ddelta[..., i:j]), _abi.view(dx[..., i:j])
-            args.dA, args.dBm = _abi.view(dA[i:j]), _abi.view(gB)
-            nbytes = lib.ssm_disc_workspace_bytes(ctypes.byref(args))
+        for i, j in _cscan_channels(x, N, d_block, True):
+            gB, gC = torch.empty_like(Bm), torch.empty_like(Cm)
+            xb, db, yb = (_steps_fit(t[..., i:j]) for t in (x, delta, dy))
+            args = _cscan_args(xb, db, A, Bm, Cm, h0, saved, i, j, method, algo)
+            args.dy, args.dlast = _abi.view(yb), _abi.view(None if dlast is None else dlast[:, i:j])
+            args.dx, args.ddelta = _abi.view(dx[..., i:j]), _abi.view(ddelta[..., i:j])
+            args.dA, args.dBm, args.dCm = _abi.view(dA[i:j]), _abi.view(gB), _abi.view(gC)
+            args.dh0 = _abi.view(None if dh0 is None else dh0[:, i:j])
+            nbytes = lib.ssm_cscan_workspace_bytes(ctypes.byref(args))
             if nbytes < 0:
-                _abi.check(lib.ssm_disc_check(ctypes.byref(args)), "ssm_disc_bwd")
-            ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
+                _abi.check(lib.ssm_cscan_check(ctypes.byref(args)), "ssm_cscan_bwd")
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-            _launch("ssm_disc_bwd", lib.ssm_disc_bwd, args, dev)
-            dBm += gB
-            del da, lam, ws
+            _launch("ssm_cscan_bwd", lib.ssm_cscan_bwd, args, x.device)
+            if dBm is None:
+                dBm, dCm = gB, gC
+            else:
+                dBm += gB
+                dCm += gC
+            del ws
         return dx, ddelta, dA, dBm, dCm, dh0, None, None, None, None
 
 

@@ -1,0 +1,68 @@
+"""GPU: the composed selective scan's kernels at their edges -- lengths around one time tile (64
+steps; 16 for float64 Hillis-Steele) and one row lane (8), every state padding and state counts
+that fill none, channels that fill no workgroup, storage orders, a broadcast A, channel tiles of
+the backward -- against the float64 oracle."""
+
+import pytest
+import torch
+
+from ssm_scan import scan as S
+from test_gpu_scan import ALGOS, _oracle_sel, close, sel_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(scan, method, ins, dy, dlast, dtype, d_block=None, prep=lambda name, t: t):
+    names = ("x", "delta", "A", "Bm", "Cm", "h0")
+    leaves = [None if t is None else prep(n, t.to("cuda", dtype)).detach().requires_grad_()
+              for n, t in zip(names, ins)]
+    y, last = S.selective_scan(*leaves, method=method, scan=scan, d_block=d_block)
+    live = [t for t in leaves if t is not None]
+    grads = torch.autograd.grad((y, last), live, (prep("dy", dy.to("cuda", dtype)), dlast.to("cuda", dtype)))
+    ry, rlast, rg = _oracle_sel(ins, method, dy, dlast, dtype)
+    close(y.detach(), ry, dtype, "y")
+    close(last.detach(), rlast, dtype, "last")
+    for name, g in zip(("dx", "ddelta", "dA", "dB", "dC", "dh0"), grads):
+        close(g, rg[name], dtype, name)
+
+
+def _problem(B, L, D, N, h0, seed):
+    g = torch.Generator().manual_seed(seed)
+    return (sel_inputs(B=B, L=L, D=D, N=N, seed=seed, h0=h0), torch.randn(B, L, D, generator=g, dtype=torch.float64),
+            torch.randn(B, D, N, generator=g, dtype=torch.float64))
+
+
+# (L, D, N): L around the row lane and the tile; N of every padding (8, 16, 32, 64) and between; D
+# below, at and past the 64 / NP channels of a workgroup
+EDGES = [(1, 1, 1), (7, 5, 3), (8, 8, 8), (9, 9, 5), (63, 4, 16), (64, 3, 16), (65, 5, 12), (15, 2, 32), (16, 3, 32),
+         (17, 1, 20), (64, 2, 64), (66, 1, 40), (129, 33, 16)]
+
+
+@pytest.mark.parametrize("edge", EDGES, ids=str)
+@pytest.mark.parametrize("scan", ALGOS)
+def test_edges_float64(scan, edge):
+    L, D, N = edge
+    for method, h0 in (("zoh", True), ("bilinear", False), ("euler", True)):
+        _run(scan, method, *_problem(2, L, D, N, h0, L + N), torch.float64)
+
+
+@pytest.mark.parametrize("scan", ALGOS)
+@pytest.mark.parametrize("shape", [(3, 70, 6, 16), (1, 150, 17, 8), (2, 65, 4, 48)], ids=str)
+def test_edges_float32(scan, shape):
+    _run(scan, "zoh", *_problem(*shape, True, 11), torch.float32)
+
+
+@pytest.mark.parametrize("scan", ALGOS)
+def test_storage_orders_and_channel_tiles(scan):
+    ins, dy, dlast = _problem(2, 75, 21, 16, True, 5)
+    ins = list(ins)
+    ins[2] = ins[2][:, :1].expand(-1, 16)       # one decay per channel shared by the states
+
+    def prep(name, t):
+        if name in ("x", "dy", "Bm"):            # (B, C, L) storage
+            return t.transpose(1, 2).contiguous().transpose(1, 2)
+        if name in ("delta", "Cm"):              # a view into a wider row
+            return torch.stack([t, t], -1).flatten(2)[..., ::2]
+        return t[:, :1].expand(-1, t.shape[1]) if name == "A" else t
+
+    _run(scan, "zoh", ins, dy, dlast, torch.float64, d_block=6, prep=prep)
