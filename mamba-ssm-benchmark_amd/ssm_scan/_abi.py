@@ -214,6 +214,26 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The binding of the launches (ssm_scan._ssmhost: checks, allocation and argument structs in
+    one native call each); raises if it is not built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _ssmhost
+        except ImportError as e:
+            raise RuntimeError("ssm_scan/_ssmhost.so is missing or does not load: build it with "
+                               "__graft_entry__.build() (make -C mamba-ssm-benchmark_amd/csrc)") from e
+        if _ssmhost.abi_version() != ABI_VERSION:
+            raise RuntimeError(f"_ssmhost ABI version {_ssmhost.abi_version()} != expected {ABI_VERSION}")
+        _host = _ssmhost
+    return _host
+
+
 _ERRORS = {EINVAL: ValueError, EKEY: KeyError, ESPACE: ValueError, EHIP: RuntimeError}
 
 

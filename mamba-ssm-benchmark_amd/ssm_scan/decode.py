@@ -85,7 +85,12 @@ class FastDecoder:
                 L["w_in4"] = _four_k(L["w_in"])
                 L["w_out4"] = _four_k(m.out_proj.weight)
         if self.path == "stack":  # the head with the final RMSNorm weight folded into its columns
-            self.head_w4 = _four_k(self.model.head.weight * self.model.norm_f.weight[None, :])
+            head_w4 = _four_k(self.model.head.weight * self.model.norm_f.weight[None, :])
+            m, (V, dm) = self.layers[0]["mixer"], self.model.head.weight.shape
+            names = ("w_in4", "conv_w", "conv_b", "x_proj_wt", "dt_proj_w", "dt_bias", "A_log", "Dskip", "w_out4")
+            self.plan = _abi.host().DecodePlan([([L[k] for k in names], L["eps"]) for L in self.layers], head_w4, dm,
+                                               m.d_inner, m.d_state, m.d_conv, m.dt_rank, V,
+                                               METHODS[m.discretization], self.model.norm_f.eps)
 
     def _layer(self, L, u, state):
         m = L["mixer"]
@@ -110,45 +115,17 @@ class FastDecoder:
     def _stack(self, tok, states):
         """The whole token step in one call: embedding rows, every block, the final norm and
         the head; returns the logits."""
-        m = self.layers[0]["mixer"]
-        B, dm, V = tok.numel(), self.model.head.weight.shape[1], self.model.head.weight.shape[0]
-        tok = tok.reshape(-1).to(torch.long).contiguous()  # a strided view of ids is copied
-        u = torch.empty(B, dm, dtype=torch.float32, device=tok.device)
-        logits = torch.empty(B, V, dtype=torch.float32, device=tok.device)
-        n = len(self.layers)
-        blocks = (_abi.DecodeBlock * n)()
-        for i, (L, st) in enumerate(zip(self.layers, states)):
-            k = blocks[i]
-            k.w_in4, k.conv_w, k.conv_b = L["w_in4"].data_ptr(), L["conv_w"].data_ptr(), L["conv_b"].data_ptr()
-            k.x_proj_wt, k.dt_proj_w = L["x_proj_wt"].data_ptr(), L["dt_proj_w"].data_ptr()
-            k.dt_bias, k.A_log, k.Dskip = L["dt_bias"].data_ptr(), L["A_log"].data_ptr(), L["Dskip"].data_ptr()
-            k.w_out4 = L["w_out4"].data_ptr()
-            k.conv_state, k.ssm_state = st.conv.data_ptr(), st.ssm.data_ptr()
-            k.eps = L["eps"]
-        a = _abi.DecodeStackArgs()
-        a.batch, a.dim, a.dstate, a.width = u.shape[0], m.d_inner, m.d_state, m.d_conv
-        a.dt_rank, a.d_model = m.dt_rank, u.shape[1]
-        a.method = METHODS[m.discretization]
-        a.conv_state_dtype = _abi.DTYPE_CODE[states[0].conv.dtype]
-        a.n_blocks = n
-        a.blocks = blocks
-        a.u = u.data_ptr()
-        a.tokens, a.embed = tok.data_ptr(), self.model.embed.weight.data_ptr()
-        a.head_w4, a.logits, a.vocab = self.head_w4.data_ptr(), logits.data_ptr(), V
-        a.head_eps = self.model.norm_f.eps
-        lib = _abi.lib()
-        need = lib.ssm_decode_stack_workspace_bytes(ctypes.byref(a))
-        key = (u.device, need)
+        conv, ssm = [s.conv for s in states], [s.ssm for s in states]
+        B = tok.numel()
+        need = self.plan.workspace_bytes(B)
+        key = (tok.device, need)
         if key not in self._ws:
-            ws = torch.empty(need, dtype=torch.uint8, device=u.device)
-            off = lib.ssm_decode_stack_status_offset(ctypes.byref(a))
+            ws = torch.empty(need, dtype=torch.uint8, device=tok.device)
+            off = self.plan.status_offset(B)
             status = ws[off:off + 4].view(torch.int32)
             status.zero_()            # the library sets it, never clears it
             self._ws[key] = (ws, status)
-        ws = self._ws[key][0]
-        a.workspace, a.workspace_bytes = ws.data_ptr(), need
-        _abi.check(lib.ssm_decode_stack(ctypes.byref(a), _abi.stream_handle(u.device)), "ssm_decode_stack")
-        return logits
+        return self.plan.step(tok, conv, ssm, self.model.embed.weight, self._ws[key][0])
 
     def _check(self, tok, states):
         """Host-side checks before any launch: the kernels size every state buffer from the
@@ -206,6 +183,11 @@ class FastDecoder:
         The decode GEMMs are skinny (B rows); they are issued through rocBLAS, whose kernels
         for these shapes take a fraction of hipBLASLt's (torch's default), and torch's choice
         is restored afterwards."""
+        if self.path == "stack":
+            self.plan.check_states(tok, [s.conv for s in states], [s.ssm for s in states])
+            if check_ids:
+                self._check_ids(tok)
+            return self._stack(tok, states)
         self._check(tok, states)
         if check_ids:
             self._check_ids(tok)
@@ -213,10 +195,6 @@ class FastDecoder:
         torch.backends.cuda.preferred_blas_library("cublas")   # rocBLAS on ROCm
         try:
             with torch.autocast(device_type="cuda", enabled=False):
-                if self.path == "stack":
-                    if len({s.conv.dtype for s in states}) != 1:
-                        raise ValueError("the stack path needs one conv state dtype for every block")
-                    return self._stack(tok, states)
                 u = self.model.embed(tok.reshape(-1))      # a fresh buffer, updated in place
                 for L, s in zip(self.layers, states):
                     u = self._layer(L, u, s)

@@ -31,14 +31,15 @@ class KernelTimer:
         return {k: [s.elapsed_time(e) for s, e in v] for k, v in self.records.items()}
 
 
-def timed_launch(name, stream, fn):
+def timed_launch(name, fn, *args):
+    """fn(*args), which issues one launch (its result passes through)."""
     t = _active
     if t is None:
-        return fn()
+        return fn(*args)
     start = torch.cuda.Event(enable_timing=True)
     end = torch.cuda.Event(enable_timing=True)
     start.record()
-    rc = fn()
+    res = fn(*args)
     end.record()
     t.records.setdefault(name, []).append((start, end))
-    return rc
+    return res

@@ -25,7 +25,7 @@ import ctypes
 import torch
 
 from . import _abi, plan
-from .hip_scan import METHODS, FusedSelectiveScanFn, _check_shapes, _require_gpu
+from .hip_scan import METHODS, FusedSelectiveScanFn, _require_gpu, check_operands
 from .profiling import timed_launch
 
 DISCRETIZATIONS = ("zoh", "euler", "bilinear")      # models/scan.py:36
@@ -54,7 +54,7 @@ def _ct(*ts):
 def _launch(name, fn, args, dev):
     with _abi.on_device(dev):
         stream = _abi.stream_handle(dev)
-        rc = timed_launch(name, stream, lambda: fn(ctypes.byref(args), stream))
+        rc = timed_launch(name, fn, ctypes.byref(args), stream)
     _abi.check(rc, name)
 
 
@@ -117,8 +117,7 @@ def discretize(delta, A, Bm, x, method="zoh"):
     Differentiable in all four tensors."""
     if method not in DISCRETIZATIONS:
         raise ValueError(f"unknown discretization {method!r}")
-    _require_gpu(delta, A, Bm, x)
-    _check_shapes(x, delta, A, Bm, Bm, None, None, None, None)  # the kernels index by (B, L, D, N)
+    check_operands(x, delta, A, Bm, Bm, None, None, None, None)  # the kernels index by (B, L, D, N)
     ct = _ct(delta, A, Bm, x)
     return DiscretizeFn.apply(delta.to(ct), A.to(ct), Bm.to(ct), x.to(ct), method)
 
@@ -137,54 +136,18 @@ class LinearScanFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, a, b, h0, algo, chunk, reverse):
-        Bsz, L, M = a.shape
-        h = torch.empty((Bsz, L, M), dtype=a.dtype, device=a.device)
-        args = _abi.LscanArgs()
-        _lscan_common(args, a, algo, chunk, reverse)
-        args.a, args.b, args.h0, args.h = (_abi.view(t) for t in (a, b, h0, h))
-        lib = _abi.lib()
-        nbytes = lib.ssm_lscan_workspace_bytes(ctypes.byref(args))
-        if nbytes < 0:
-            _abi.check(lib.ssm_lscan_check(ctypes.byref(args)), "ssm_lscan")
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=a.device) if nbytes else None
-        if ws is not None:
-            args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-        _launch("ssm_lscan", lib.ssm_lscan, args, a.device)
+        cfg = (algo, int(chunk or 0), bool(reverse))
+        h = timed_launch("ssm_lscan", _abi.host().lscan_forward, a, b, h0, *cfg)
         ctx.save_for_backward(a, h0, h)
-        ctx.cfg = (algo, chunk, reverse)
+        ctx.cfg = cfg
         return h
 
     @staticmethod
     def backward(ctx, dh):
         a, h0, h = ctx.saved_tensors
-        algo, chunk, reverse = ctx.cfg
-        da, db = torch.empty_like(h), torch.empty_like(h)
-        dh0 = torch.empty_like(h0) if h0 is not None and ctx.needs_input_grad[2] else None
-        lscan_bwd(a, h0, h, dh, da, db, dh0, algo, chunk, reverse)
+        da, db, dh0 = timed_launch("ssm_lscan_bwd", _abi.host().lscan_backward, a, h0, h, dh, *ctx.cfg,
+                                   ctx.needs_input_grad[2])
         return da, db, dh0, None, None, None
-
-
-def _lscan_common(args, a, algo, chunk, reverse):
-    Bsz, L, M = a.shape
-    args.batch, args.seqlen, args.width = Bsz, L, M
-    args.algo, args.dtype, args.reverse = algo, _abi.DTYPE_CODE[a.dtype], int(bool(reverse))
-    args.chunk = int(chunk or 0)
-
-
-def lscan_bwd(a, h0, h, dh, da, db, dh0, algo, chunk=None, reverse=False):
-    """Adjoint of a linear scan into preallocated (B, L, M) da, db (= lambda) and (B, M) dh0."""
-    args = _abi.LscanBwdArgs()
-    _lscan_common(args, a, algo, chunk, reverse)
-    args.a, args.h0, args.h, args.dh = (_abi.view(t) for t in (a, h0, h, dh))
-    args.da, args.db, args.dh0 = (_abi.view(t) for t in (da, db, dh0))
-    lib = _abi.lib()
-    nbytes = lib.ssm_lscan_bwd_workspace_bytes(ctypes.byref(args))
-    if nbytes < 0:
-        _abi.check(lib.ssm_lscan_bwd_check(ctypes.byref(args)), "ssm_lscan_bwd")
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=a.device) if nbytes else None
-    if ws is not None:
-        args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-    _launch("ssm_lscan_bwd", lib.ssm_lscan_bwd, args, a.device)
 
 
 def _scan(name, a, b, h0=None, chunk_size=None, reverse=False):
@@ -242,42 +205,6 @@ def _scan_algo(name):
 
 
 # ------------------------------------------------------------------ composed selective scan
-_CSCAN_WORKSPACE = 1 << 28   # bytes of dB / dC partials per backward launch
-
-
-def _cscan_args(x, delta, A, Bm, Cm, h0, saved, i, j, method, algo):
-    """The operands both directions share; x and delta are channels i..j already, the rest whole."""
-    args = _abi.CscanArgs()
-    args.batch, args.seqlen, args.dim, args.dstate = *x.shape, A.shape[1]
-    args.algo, args.method, args.dtype = algo, METHODS[method], _abi.DTYPE_CODE[x.dtype]
-    args.x, args.delta, args.A = _abi.view(x), _abi.view(delta), _abi.view(A[i:j])
-    args.Bm, args.Cm = _abi.view(Bm), _abi.view(Cm)
-    args.h0 = _abi.view(None if h0 is None else h0[:, i:j])
-    if saved is not None:
-        args.saved = _abi.Tensor(saved[:, :, i:j].data_ptr(), saved.stride()[:3])
-    return args
-
-
-def _cscan_channels(x, N, d_block, workspace):
-    """Channel tiles of the launches: those of d_block, else all channels at once up to 2^21 and,
-    with `workspace`, as many as keep the backward's partials (2 x L x NP per 64 / NP channels and
-    batch row) within _CSCAN_WORKSPACE."""
-    Bsz, L, D = x.shape
-    step = 1 << 21
-    if d_block and d_block > 0:
-        step = min(step, d_block)
-    elif workspace and N <= 64:
-        NP = max(8, 1 << (N - 1).bit_length())
-        step = min(step, max(1, _CSCAN_WORKSPACE // (Bsz * L * 2 * NP * x.element_size())) * (64 // NP))
-    return [(i, min(D, i + step)) for i in range(0, D, step)]
-
-
-def _steps_fit(t):
-    """t, or a contiguous copy where 64 steps of a batch row span 2 GiB (the kernels' offsets)."""
-    fits = (t.stride(2) * (t.shape[2] - 1) + 63 * t.stride(1) + 1) * t.element_size() < 1 << 31
-    return t if fits else t.contiguous()
-
-
 class SelectiveScanFn(torch.autograd.Function):
     """y, last = selective scan by a named algorithm (models/scan.py:193-255).
 
@@ -285,8 +212,8 @@ class SelectiveScanFn(torch.autograd.Function):
     (B, L, D, N) tensor exists; saved for the backward are x, delta, A, Bm, Cm, h0 and the state
     entering every time tile.  The backward recomputes the states tile by tile, runs the adjoint
     scan lambda_t = g_t + a_{t+1} lambda_{t+1} with the same algorithm and maps (da, db) =
-    (lambda h_{t-1}, lambda) back through the discretization, in channel tiles of d_block
-    (default: _CSCAN_WORKSPACE).  chunk_size is the chunk of the linear scan over materialized
+    (lambda h_{t-1}, lambda) back through the discretization, in channel tiles of d_block (default:
+    as many channels as keep the workspace within 256 MiB).  chunk_size is the chunk of the linear scan over materialized
     tensors; here a chunk is a wavefront's part of a time tile."""
 
     @staticmethod
@@ -297,58 +224,17 @@ class SelectiveScanFn(torch.autograd.Function):
         chunk = int(chunk_size or 0)
         if not 0 <= chunk < 1 << 30:
             raise ValueError(f"chunk={chunk} out of range")
-        Bsz, L, D = x.shape
-        N = A.shape[1]
-        Bm, Cm = _steps_fit(Bm), _steps_fit(Cm)
-        y = torch.empty_like(x)
-        last = torch.empty(Bsz, D, N, dtype=x.dtype, device=x.device)
-        lib = _abi.lib()
-        saved = None
-        if any(ctx.needs_input_grad[:6]):
-            tile = lib.ssm_cscan_tile(algo, _abi.DTYPE_CODE[x.dtype])
-            saved = torch.empty(Bsz, -(-L // tile), D, N, dtype=x.dtype, device=x.device)
-        for i, j in _cscan_channels(x, N, None, False):
-            xb, db = _steps_fit(x[..., i:j]), _steps_fit(delta[..., i:j])
-            args = _cscan_args(xb, db, A, Bm, Cm, h0, saved, i, j, method, algo)
-            args.y, args.last = _abi.view(y[..., i:j]), _abi.view(last[:, i:j])
-            _launch("ssm_cscan_fwd", lib.ssm_cscan_fwd, args, x.device)
+        y, last, Bm, Cm, saved = timed_launch("ssm_cscan_fwd", _abi.host().cscan_forward, x, delta, A, Bm, Cm, h0, algo,
+                                              METHODS[method], any(ctx.needs_input_grad[:6]))
         ctx.save_for_backward(x, delta, A, Bm, Cm, h0, saved)
         ctx.set_materialize_grads(False)   # an unused output passes None (no zero fill)
-        ctx.cfg = (method, algo, d_block)
+        ctx.cfg = (algo, METHODS[method], int(d_block or 0))
         return y, last
 
     @staticmethod
     def backward(ctx, dy, dlast):
-        x, delta, A, Bm, Cm, h0, saved = ctx.saved_tensors
-        method, algo, d_block = ctx.cfg
-        N = A.shape[1]
-        if dy is None:
-            dy = torch.zeros_like(x)
-        dx, ddelta, dA = torch.empty_like(x), torch.empty_like(delta), torch.empty_like(A)
-        dBm = dCm = None
-        dh0 = None if h0 is None else torch.empty_like(h0)
-        lib = _abi.lib()
-        for i, j in _cscan_channels(x, N, d_block, True):
-            gB, gC = torch.empty_like(Bm), torch.empty_like(Cm)
-            xb, db, yb = (_steps_fit(t[..., i:j]) for t in (x, delta, dy))
-            args = _cscan_args(xb, db, A, Bm, Cm, h0, saved, i, j, method, algo)
-            args.dy, args.dlast = _abi.view(yb), _abi.view(None if dlast is None else dlast[:, i:j])
-            args.dx, args.ddelta = _abi.view(dx[..., i:j]), _abi.view(ddelta[..., i:j])
-            args.dA, args.dBm, args.dCm = _abi.view(dA[i:j]), _abi.view(gB), _abi.view(gC)
-            args.dh0 = _abi.view(None if dh0 is None else dh0[:, i:j])
-            nbytes = lib.ssm_cscan_workspace_bytes(ctypes.byref(args))
-            if nbytes < 0:
-                _abi.check(lib.ssm_cscan_check(ctypes.byref(args)), "ssm_cscan_bwd")
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-            args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-            _launch("ssm_cscan_bwd", lib.ssm_cscan_bwd, args, x.device)
-            if dBm is None:
-                dBm, dCm = gB, gC
-            else:
-                dBm += gB
-                dCm += gC
-            del ws
-        return dx, ddelta, dA, dBm, dCm, dh0, None, None, None, None
+        grads = timed_launch("ssm_cscan_bwd", _abi.host().cscan_backward, *ctx.saved_tensors, *ctx.cfg, dy, dlast)
+        return (*grads, None, None, None, None)
 
 
 def selective_scan_reference(x, delta, A, Bm, Cm, h0=None, method="zoh"):
@@ -358,8 +244,7 @@ def selective_scan_reference(x, delta, A, Bm, Cm, h0=None, method="zoh"):
     in every lane -- the same recurrence as the reference's loop, without storing the states."""
     if method not in DISCRETIZATIONS:
         raise ValueError(f"unknown discretization {method!r}")
-    _require_gpu(x, delta, A, Bm, Cm, h0)
-    _check_shapes(x, delta, A, Bm, Cm, None, None, None, h0)
+    check_operands(x, delta, A, Bm, Cm, None, None, None, h0)
     return FusedSelectiveScanFn.apply(x, delta, A, Bm, Cm, None, None, None, h0, METHODS[method], False)
 
 
@@ -389,6 +274,6 @@ def selective_scan(x, delta, A, Bm, Cm, h0=None, method="zoh", scan="chunked",
         if scan == "reference":
             y, last = selective_scan_reference(*args, method=method)
         else:
-            _check_shapes(*args[:5], None, None, None, args[5])
+            check_operands(*args[:5], None, None, None, args[5])
             y, last = SelectiveScanFn.apply(*args, method, scan, d_block, chunk_size)
     return y.to(dtype), last
