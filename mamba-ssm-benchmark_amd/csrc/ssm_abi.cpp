@@ -1001,7 +1001,6 @@ static ConvParams conv_params(const ssm_conv_args *a) {
   ConvParams p;
   memset(&p, 0, sizeof(p));
   p.B = a->batch; p.L = a->seqlen; p.D = a->dim; p.W = a->width;
-  p.TB = kConvTT;
   p.nblk = (int)cdiv(a->seqlen, kConvTB);
   p.silu = a->silu != 0;
   p.has_bias = has(a->bias); p.has_sin = has(a->state_in); p.has_sout = has(a->state_out);

@@ -207,16 +207,15 @@ struct CscParams {
 };
 hipError_t launch_csc(const CscParams &p, int algo, int dtype, int method, int np, bool bwd, hipStream_t s);
 
-// Causal depthwise conv over (B, L, D) views; a lane owns (b, d, one block of TB steps).
-// Causal conv: a workgroup covers kConvDG channels x kConvTG lanes of kConvTT time steps
-// (kConvTT >= W - 1 for every width <= 8).
+// Causal depthwise conv over (B, L, D) views: a workgroup covers kConvDG channels x kConvTG
+// wavefronts of kConvTT time steps (kConvTT >= W - 1 for every width <= 8).
 constexpr int kConvTT = 8, kConvTG = 4, kConvDG = 64;
 struct ConvParams {
   int64_t B, L, D, W;
-  int nblk, TB;  // time blocks of kConvTG * kConvTT steps (one workgroup row each), kConvTT
+  int nblk;  // workgroups along time: kConvTG * kConvTT steps each
   int silu, has_bias, has_sin, has_sout, has_dbias;
   KView x, w, bias, sin, out, sout, dout, dx, dw, dbias;  // sin / sout: (B, D, W-1)
-  void *ws;  // backward: (B * nblk, D, W + 1) partial dweight / dbias, one row per workgroup
+  void *ws;  // backward: (B * nblk, W + 1, D) partial dweight / dbias, one row per workgroup
 };
 
 // RMSNorm over rows of C <= kNormMaxC elements (unit column stride): a wavefront per row,
