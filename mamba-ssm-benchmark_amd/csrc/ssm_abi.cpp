@@ -1068,8 +1068,6 @@ static NormParams norm_params(const ssm_norm_args *a) {
   p.dy = a->dout.data; p.sdy = a->dout.stride[0];
   p.dx = a->dx.data; p.sdx = a->dx.stride[0];
   p.dw = a->dweight;
-  p.rpw = norm_rows_per_wave(norm_kc_of(a->dim));
-  p.nblk = cdiv(a->rows, (int64_t)kNormWaves * p.rpw);
   return p;
 }
 
@@ -1097,8 +1095,7 @@ int ssm_norm_check(const ssm_norm_args *a) {
 
 int64_t ssm_norm_workspace_bytes(const ssm_norm_args *a) {
   if (ssm_norm_check(a)) return -1;
-  const NormParams p = norm_params(a);
-  return align256(p.nblk * a->dim * state_size(a->dtype));
+  return align256(std::min<int64_t>(cdiv(a->rows, norm_bwd_rows(a->dim)), kNormBlocks) * a->dim * state_size(a->dtype));
 }
 
 int ssm_norm_fwd(const ssm_norm_args *a, void *stream) {

@@ -218,14 +218,12 @@ struct ConvParams {
   void *ws;  // backward: (B * nblk, W + 1, D) partial dweight / dbias, one row per workgroup
 };
 
-// RMSNorm over rows of C <= kNormMaxC elements (unit column stride): a wavefront per row,
-// kNormWaves wavefronts per workgroup; the backward's wavefronts take norm_rows_per_wave rows.
-constexpr int kNormWaves = 4, kNormThreads = kNormWaves * 64, kNormFinThreads = 1024, kNormMaxC = 1024;
-// columns per lane (power of two) for a row of C elements
-inline constexpr int norm_kc_of(int64_t C) {
-  return C <= 64 ? 1 : C <= 128 ? 2 : C <= 256 ? 4 : C <= 512 ? 8 : C <= 1024 ? 16 : 0;
-}
-inline constexpr int norm_rows_per_wave(int kc) { return kc <= 4 ? 8 : kc == 8 ? 4 : 2; }
+// RMSNorm over rows of C <= kNormMaxC elements (unit column stride).  A backward workgroup takes at
+// least norm_bwd_rows(C) rows and leaves one partial row of dw; at most kNormBlocks of them run (two
+// per CU: the wavefronts that fit at once), more only add partial rows.
+constexpr int kNormThreads = 256, kNormBwdThreads = 512, kNormFinThreads = 1024, kNormMaxC = 1024;
+constexpr int kNormBlocks = 512;
+inline constexpr int norm_bwd_rows(int64_t C) { return C <= 256 ? 32 : C <= 512 ? 16 : 8; }
 struct NormParams {
   int64_t R, C;
   double eps;
@@ -234,7 +232,6 @@ struct NormParams {
   void *y, *rstd, *dx, *dw;
   void *ws;      // backward: (nblk, C) per-workgroup weight-gradient partials
   int64_t nblk;  // backward workgroups
-  int rpw;       // backward rows per wavefront
 };
 
 // Fused decode layer (float32, row-major); one workgroup per batch row.
