@@ -207,10 +207,19 @@ struct TileIn {
   }
 };
 
+// The last row of each array stays zero: lanes of no channel or no state (pad lanes) read it, so that
+// every one of their steps is the identity whatever the operands of the lanes beside them hold.  (The
+// row is picked once; with B = C = 0 alone an infinite x, or a growing decay exp(-delta), gave 0 * inf.)
 template <typename CT, int R, int NP, bool BWD>
 struct StageLds {
   static constexpr int CW = kWave / NP, RP = R + 16 / (int)sizeof(CT);
-  CT x[CW][RP], dt[CW][RP], g[BWD ? CW : 1][RP], B[NP][RP], C[NP][RP];
+  CT x[CW + 1][RP], dt[CW + 1][RP], g[BWD ? CW + 1 : 1][RP], B[NP + 1][RP], C[NP + 1][RP];
+  __device__ __forceinline__ void clear_pad(int lane) {
+    if (lane < RP) {
+      x[CW][lane] = dt[CW][lane] = B[NP][lane] = C[NP][lane] = 0;
+      if constexpr (BWD) g[CW][lane] = 0;
+    }
+  }
 };
 
 template <typename CT, int NP, int METHOD, int ALGO>
@@ -226,6 +235,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
   const int L = (int)p.L, D = (int)p.D, N = (int)p.N;
   const bool valid = d < D && n < N;
   const AConst<CT> ac = make_aconst(valid ? vload<CT>(p.A, d * p.A.s0 + n * p.A.s1) : (CT)-1);
+  const int cr = valid ? c : CW, nr = valid ? n : NP;  // rows of the staged operands
   const TileIn<CT, R, CW> ix(p.x, b, d0, D, ST, lane), id(p.dt, b, d0, D, ST, lane);
   const TileIn<CT, R, NP> iB(p.Bm, b, 0, N, ST, lane), iC(p.Cm, b, 0, N, ST, lane);
   CT carry = p.h0.p && valid ? vload<CT>(p.h0, b * p.h0.s0 + d * p.h0.s1 + n * p.h0.s2) : (CT)0;
@@ -238,6 +248,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
     iC.load(nC, t0, nv, lane);
   };
   fetch(0);
+  S.clear_pad(lane);
   int buf = 0, i = 0;
   const int yi = state_index<NP, R>(lane);
   const bool yown = state_owner<NP, R>(lane) && d < D;
@@ -251,10 +262,10 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
     wave_lds_sync();
     if (base + T < L) fetch(base + T);
     CT a[R], h[R], y[R], x[R], dt[R], Bv[R];
-    lds_row(&S.dt[c][0], dt);
-    lds_row(&S.x[c][0], x);
-    lds_row(&S.B[n][0], Bv);
-    lds_row(&S.C[n][0], y);
+    lds_row(&S.dt[cr][0], dt);
+    lds_row(&S.x[cr][0], x);
+    lds_row(&S.B[nr][0], Bv);
+    lds_row(&S.C[nr][0], y);
 #pragma unroll
     for (int r = 0; r < R; ++r) {  // a zero step is the identity
       CT coef;
@@ -291,6 +302,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
   const int L = (int)p.L, D = (int)p.D, N = (int)p.N;
   const bool valid = d < D && n < N;
   const AConst<CT> ac = make_aconst(valid ? vload<CT>(p.A, d * p.A.s0 + n * p.A.s1) : (CT)-1);
+  const int cr = valid ? c : CW, nr = valid ? n : NP;  // rows of the staged operands
   const TileIn<CT, R, CW> ix(p.x, b, d0, D, ST, lane), id(p.dt, b, d0, D, ST, lane), ig(p.dy, b, d0, D, ST, lane);
   const TileIn<CT, R, NP> iB(p.Bm, b, 0, N, ST, lane), iC(p.Cm, b, 0, N, ST, lane);
   // mu: the adjoint entering the tile's last step from the steps after it
@@ -307,6 +319,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
   };
   const int nt = (L + T - 1) / T;
   fetch(nt - 1);
+  S.clear_pad(lane);
   int buf = 0;
   double gA = 0;
   const int oi = state_index<NP, V>(lane), wi = chan_index<NP, V>(lane);
@@ -324,11 +337,11 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
     wave_lds_sync();
     if (i > 0) fetch(i - 1);
     CT a[R], a0[R], coef[R], h[R], dt[R], x[R], Bv[R], dy[R], g[R];
-    lds_row(&S.dt[c][0], dt);
-    lds_row(&S.x[c][0], x);
-    lds_row(&S.B[n][0], Bv);
-    lds_row(&S.g[c][0], dy);
-    lds_row(&S.C[n][0], g);
+    lds_row(&S.dt[cr][0], dt);
+    lds_row(&S.x[cr][0], x);
+    lds_row(&S.B[nr][0], Bv);
+    lds_row(&S.g[cr][0], dy);
+    lds_row(&S.C[nr][0], g);
 #pragma unroll
     for (int r = 0; r < R; ++r) {  // a zero step is the identity
       g[r] *= dy[r];

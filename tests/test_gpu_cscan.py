@@ -66,3 +66,47 @@ def test_storage_orders_and_channel_tiles(scan):
         return t[:, :1].expand(-1, t.shape[1]) if name == "A" else t
 
     _run(scan, "zoh", ins, dy, dlast, torch.float64, d_block=6, prep=prep)
+
+
+def _close_norm(got, ref, name):
+    """float32 sums of a few hundred terms: 2-norm of the difference within 2e-5 of the result's."""
+    got, ref = got.detach().double().cpu(), torch.as_tensor(ref)
+    assert bool(torch.isfinite(got).all()), f"{name} is not finite"
+    assert float((got - ref).norm()) <= 2e-5 * float(ref.norm()) + 1e-30, (name, float((got - ref).norm()), float(ref.norm()))
+
+
+def _check_all(scan, method, ins, dy, dlast, ref_ins=None):
+    leaves = [None if t is None else t.float().cuda().requires_grad_() for t in ins]
+    y, last = S.selective_scan(*leaves, method=method, scan=scan)
+    grads = torch.autograd.grad((y, last), [t for t in leaves if t is not None], (dy.float().cuda(), dlast.float().cuda()))
+    ry, rlast, rg = _oracle_sel(ref_ins or ins, method, dy, dlast, torch.float32)
+    _close_norm(y, ry, "y")
+    _close_norm(last, rlast, "last")
+    for name, g in zip(("dx", "ddelta", "dA", "dB", "dC", "dh0"), grads):
+        _close_norm(g, rg[name], name)
+
+
+@pytest.mark.parametrize("N", [5, 12, 20, 33])
+@pytest.mark.parametrize("scan", ALGOS)
+def test_pad_states_with_negative_steps(scan, N):
+    """A > 0 and delta < 0 decay; a pad lane of its own decay would grow past float32 within 8 steps."""
+    ins, dy, dlast = _problem(2, 75, 6, N, True, N)
+    ins = list(ins)
+    g = torch.Generator().manual_seed(N)
+    ins[1] = -10 - 4 * torch.rand(2, 75, 6, generator=g, dtype=torch.float64)
+    ins[2] = 0.005 + 0.015 * torch.rand(6, N, generator=g, dtype=torch.float64)
+    _check_all(scan, "zoh", ins, dy, dlast)
+
+
+@pytest.mark.parametrize("scan", ALGOS)
+def test_infinite_input_with_pad_states(scan):
+    """An infinite x makes its channel infinite from its step on (all B, C > 0), and nothing else."""
+    ins, _, _ = _problem(2, 75, 6, 12, True, 3)
+    x, delta, A, Bm, Cm, h0 = (t.float().cuda() for t in ins)
+    Bm, Cm, delta = Bm.abs() + 0.1, Cm.abs() + 0.1, delta * 0.1
+    want, _ = S.selective_scan(x, delta, A, Bm, Cm, h0, scan=scan)
+    x[1, 40, 2] = float("inf")
+    y, last = S.selective_scan(x, delta, A, Bm, Cm, h0, scan=scan)
+    assert bool(torch.isposinf(y[1, 40:, 2]).all()) and bool(torch.isposinf(last[1, 2]).all())
+    want[1, 40:, 2] = y[1, 40:, 2]
+    assert torch.equal(y, want)
