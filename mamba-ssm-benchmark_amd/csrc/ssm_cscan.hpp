@@ -222,6 +222,14 @@ struct StageLds {
   }
 };
 
+// A of -inf (-exp of a large A_log) as a finite value whose decay over any step is 0 too: the steps
+// past the sequence's end have delta = 0, and 0 * inf is no identity.
+template <typename CT>
+__device__ __forceinline__ CT finite_decay(CT A) {
+  const CT lim = sizeof(CT) == 8 ? (CT)-1e300 : (CT)-1e37;
+  return A < lim ? lim : A;
+}
+
 template <typename CT, int NP, int METHOD, int ALGO>
 __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const CscParams p) {
   constexpr int RL = cs_rl<CT, ALGO>(), R = cs_rows<CT, ALGO>(), T = RL * R, CW = kWave / NP;
@@ -234,7 +242,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
   const int64_t b = blockIdx.y;
   const int L = (int)p.L, D = (int)p.D, N = (int)p.N;
   const bool valid = d < D && n < N;
-  const AConst<CT> ac = make_aconst(valid ? vload<CT>(p.A, d * p.A.s0 + n * p.A.s1) : (CT)-1);
+  const AConst<CT> ac = make_aconst(valid ? finite_decay(vload<CT>(p.A, d * p.A.s0 + n * p.A.s1)) : (CT)-1);
   const int cr = valid ? c : CW, nr = valid ? n : NP;  // rows of the staged operands
   const TileIn<CT, R, CW> ix(p.x, b, d0, D, ST, lane), id(p.dt, b, d0, D, ST, lane);
   const TileIn<CT, R, NP> iB(p.Bm, b, 0, N, ST, lane), iC(p.Cm, b, 0, N, ST, lane);
@@ -301,7 +309,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
   const int64_t b = blockIdx.y;
   const int L = (int)p.L, D = (int)p.D, N = (int)p.N;
   const bool valid = d < D && n < N;
-  const AConst<CT> ac = make_aconst(valid ? vload<CT>(p.A, d * p.A.s0 + n * p.A.s1) : (CT)-1);
+  const AConst<CT> ac = make_aconst(valid ? finite_decay(vload<CT>(p.A, d * p.A.s0 + n * p.A.s1)) : (CT)-1);
   const int cr = valid ? c : CW, nr = valid ? n : NP;  // rows of the staged operands
   const TileIn<CT, R, CW> ix(p.x, b, d0, D, ST, lane), id(p.dt, b, d0, D, ST, lane), ig(p.dy, b, d0, D, ST, lane);
   const TileIn<CT, R, NP> iB(p.Bm, b, 0, N, ST, lane), iC(p.Cm, b, 0, N, ST, lane);

@@ -110,3 +110,16 @@ def test_infinite_input_with_pad_states(scan):
     assert bool(torch.isposinf(y[1, 40:, 2]).all()) and bool(torch.isposinf(last[1, 2]).all())
     want[1, 40:, 2] = y[1, 40:, 2]
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("L", [70, 128])
+@pytest.mark.parametrize("scan", ALGOS)
+def test_infinite_decay(scan, L):
+    """A = -inf (-exp of a large A_log): the state forgets at once and adds nothing, also where the
+    sequence ends inside a time tile.  The oracle takes the largest decays float32 holds for it."""
+    ins, dy, dlast = _problem(2, L, 6, 12, True, 9)
+    ins, ref = list(ins), list(ins)
+    ins[2], ref[2] = ins[2].clone(), ins[2].clone()
+    ins[2][1, 3], ins[2][4] = -float("inf"), -float("inf")
+    ref[2][1, 3], ref[2][4] = -1e38, -1e38
+    _check_all(scan, "zoh", ins, dy, dlast, ref)
