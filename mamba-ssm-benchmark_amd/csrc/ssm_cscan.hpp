@@ -168,7 +168,7 @@ struct TileIn {
   static constexpr int E = (R * COLS + kWave - 1) / kWave, RP = R + 16 / (int)sizeof(CT);
   const char *base;   // step 0, column c0 of batch row b
   int64_t s1;         // bytes between steps of the sequence
-  uint32_t off[E];    // the lane's elements; kDropOffset (reads 0) for columns past the end
+  uint32_t off[E];    // the lane's elements, below 2^31 bytes; kDropOffset (reads 0) for columns past the end
   bool tfast;
   __device__ __forceinline__ TileIn(const KView &v, int64_t b, int c0, int count, int step, int lane)
       : base((const char *)v.p + (b * v.s0 + c0 * v.s2) * (int64_t)sizeof(CT)), s1(v.s1 * (int64_t)sizeof(CT)),
@@ -184,7 +184,7 @@ struct TileIn {
   // Steps t0, t0 + step, ..; those at or past nv of the R read 0.
   __device__ __forceinline__ void load(CT (&v)[E], int t0, int nv, int lane) const {
     const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc((void *)(base + t0 * s1), (short)0, 0x7ffffff0, kBufferFlags);
+        __builtin_amdgcn_make_buffer_rsrc((void *)(base + t0 * s1), (short)0, 0x7fffffff, kBufferFlags);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       uint32_t o = off[i];

@@ -123,3 +123,20 @@ def test_infinite_decay(scan, L):
     ins[2][1, 3], ins[2][4] = -float("inf"), -float("inf")
     ref[2][1, 3], ref[2][4] = -1e38, -1e38
     _check_all(scan, "zoh", ins, dy, dlast, ref)
+
+
+def test_operand_spans_up_to_2_gib():
+    """64 steps of a batch row may span up to 2^31 bytes, the last elements included."""
+    ins, dy, dlast = _problem(1, 64, 3, 5, False, 21)
+    x, delta, A, Bm, Cm, _ = (None if t is None else t.float().cuda() for t in ins)
+    store = torch.empty(1 << 29, device="cuda")
+    for s2 in (134217726, 134217727):   # one B for every step; its last state
+        Bs = store[:4 * s2 + 1].as_strided((1, 64, 5), (0, 0, s2))  # starts 32 and 16 bytes below 2^31
+        store[:4 * s2 + 1:s2] = Bm[0, 0]
+        res = []
+        for v in (Bm[:, :1].expand(1, 64, 5).contiguous(), Bs):
+            leaves = [x.clone().requires_grad_(), v.detach().requires_grad_()]
+            y, last = S.selective_scan(leaves[0], delta, A, leaves[1], Cm, scan="chunked")
+            res.append((y, last, *torch.autograd.grad((y, last), leaves, (dy.float().cuda(), dlast.float().cuda()))))
+        for got, want in zip(res[1], res[0]):
+            assert torch.equal(got, want)
