@@ -37,7 +37,6 @@
 // 151 + 284 (with 4 row lanes 200 + 484), hillis_steele 184 + 290 (237 + 511), sequential 149 +
 // 283 (one wavefront per workgroup 185 + 467).
 #include "ssm_device.hpp"
-#include "ssm_dpp.hpp"
 #include "ssm_internal.hpp"
 #include "ssm_tiles.hpp"
 #include "ssm_tilescan.hpp"
@@ -63,25 +62,25 @@ struct Chain {
   }
   __device__ __forceinline__ int64_t h_off(int t) const { return b * P.h.s0 + (int64_t)t * P.h.s1 + m * P.h.s2; }
   // Adjoint (GRAD): the forward scan's state before the step at processing position pos -- the
-  // state at the next position, since the adjoint runs against the forward scan; h0 at the last.
-  // `v` is that state read at a clamped position (never past the sequence).
+  // state at the next position, since the adjoint runs against the forward scan; read at a clamped
+  // position, so that h0f() (read once, not in the walk) can take its place at the last one.
   __device__ __forceinline__ CT hprev_at(int pos) const {
     return vload<CT>(P.hf, b * P.hf.s0 + (int64_t)t_of(min(pos + 1, (int)P.L - 1)) * P.hf.s1 + m * P.hf.s2);
   }
-  __device__ __forceinline__ CT hprev(CT v, int pos) const {
-    if (pos + 1 < (int)P.L) return v;
+  __device__ __forceinline__ CT h0f() const {
     return P.h0f.p ? vload<CT>(P.h0f, b * P.h0f.s0 + m * P.h0f.s1) : (CT)0;
   }
   // Stores the scan's value v at position pos; with GRAD, v is lambda (= db) and da = lambda
-  // h_{prev} and, at the forward scan's first step, dh0 = a lambda go out with it.
+  // h_{prev} goes out with it.
   template <bool GRAD>
   __device__ __forceinline__ void put(int pos, CT v, CT hp) const {
     const int t = t_of(pos);
     vstore<CT>(P.h, h_off(t), v);
-    if constexpr (GRAD) {
-      vstore<CT>(P.da, b * P.da.s0 + (int64_t)t * P.da.s1 + m * P.da.s2, v * hprev(hp, pos));
-      if (pos + 1 == (int)P.L && P.dh0.p) vstore<CT>(P.dh0, b * P.dh0.s0 + m * P.dh0.s1, a_at(t) * v);
-    }
+    if constexpr (GRAD) vstore<CT>(P.da, b * P.da.s0 + (int64_t)t * P.da.s1 + m * P.da.s2, v * hp);
+  }
+  // dh0 = a lambda of the last position (the forward scan's first step).
+  __device__ __forceinline__ void put_dh0(CT v) const {
+    if (P.dh0.p) vstore<CT>(P.dh0, b * P.dh0.s0 + m * P.dh0.s1, a_at(t_of((int)P.L - 1)) * v);
   }
   __device__ __forceinline__ CT h0() const {
     return P.h0.p ? vload<CT>(P.h0, b * P.h0.s0 + m * P.h0.s1) : (CT)0;
@@ -105,6 +104,7 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
   const int L = (int)P.L;
   auto step = [&](int r) { return tile_step<ALGO, RL, R>(tr, r); };
   CT carry = ch.h0();
+  const CT hfirst = GRAD ? ch.h0f() : (CT)0;
   CT na[R], nb[R], nh[GRAD ? R : 1];
   auto fetch = [&](int base) {  // reads at clamped positions
 #pragma unroll
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
       const bool in = base + step(r) < L;
       a[r] = in ? na[r] : (CT)1;
       b[r] = in ? nb[r] : (CT)0;
-      if constexpr (GRAD) hp[r] = nh[r];
+      if constexpr (GRAD) hp[r] = base + step(r) + 1 < L ? nh[r] : hfirst;
     }
     if (base + T < L) fetch(base + T);
     CT hin;
@@ -133,6 +133,7 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
     for (int r = 0; r < R; ++r) {
       const int pos = base + step(r);
       if (mval && pos < L) ch.template put<GRAD>(pos, b[r], hp[GRAD ? r : 0]);
+      if (GRAD && mval && pos + 1 == L) ch.put_dh0(b[r]);
     }
   }
 }
@@ -150,6 +151,8 @@ constexpr int kSeqAhead = 16;  // steps whose inputs are read before their depen
 template <typename CT, bool REDUCE, bool GRAD>
 __device__ __forceinline__ void chunk_walk(const LscanParams &P, const Chain<CT> &ch, int p0, int p1, CT &h,
                                            CT &prod) {
+  const bool last = GRAD && p1 == (int)P.L;
+  const CT hfirst = last ? ch.h0f() : (CT)0;
   int pos = p0;
   for (; pos + kSeqAhead <= p1; pos += kSeqAhead) {  // inputs read ahead of the updates
     CT av[kSeqAhead], bv[kSeqAhead], hp[GRAD ? kSeqAhead : 1];
@@ -163,14 +166,17 @@ __device__ __forceinline__ void chunk_walk(const LscanParams &P, const Chain<CT>
     for (int u = 0; u < kSeqAhead; ++u) {
       h = fma(av[u], h, bv[u]);
       if constexpr (REDUCE) prod *= av[u];
-      else ch.template put<GRAD>(pos + u, h, hp[GRAD ? u : 0]);
+      else ch.template put<GRAD>(pos + u, h, last && pos + u + 1 == p1 ? hfirst : hp[GRAD ? u : 0]);
     }
   }
   for (; pos < p1; ++pos) {
     const CT a = ch.mult(pos);
     h = fma(a, h, ch.b_at(ch.t_of(pos)));
     if constexpr (REDUCE) prod *= a;
-    else ch.template put<GRAD>(pos, h, GRAD ? ch.hprev_at(pos) : (CT)0);
+    else ch.template put<GRAD>(pos, h, !GRAD ? (CT)0 : last && pos + 1 == p1 ? hfirst : ch.hprev_at(pos));
+  }
+  if constexpr (GRAD && !REDUCE) {
+    if (last) ch.put_dh0(h);
   }
 }
 
