@@ -7,7 +7,9 @@
 // in tiles; row lane tr, a wavefront, holds its steps of the tile in registers while the next
 // tile's are read.  What the tile does with them is the algorithm:
 //   sequential     models/scan.py:70-76    the row lanes take turns, each walking its 16 steps
-//                                          from the state the previous one hands over.
+//                                          from the state the previous one hands over; forward
+//                                          passes of short or wide scans run one wavefront per
+//                                          workgroup instead (k_lscan_seqt).
 //   hillis_steele  models/scan.py:87-98    recursive doubling along the tile (offsets below the
 //                                          row lanes through LDS, the others in registers); the
 //                                          state entering a tile is folded into its first
@@ -37,6 +39,7 @@
 // 151 + 284 (with 4 row lanes 200 + 484), hillis_steele 184 + 290 (237 + 511), sequential 149 +
 // 283 (one wavefront per workgroup 185 + 467).
 #include "ssm_device.hpp"
+#include "ssm_dpp.hpp"
 #include "ssm_internal.hpp"
 #include "ssm_tiles.hpp"
 #include "ssm_tilescan.hpp"
@@ -105,15 +108,18 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
   auto step = [&](int r) { return tile_step<ALGO, RL, R>(tr, r); };
   CT carry = ch.h0();
   const CT hfirst = GRAD ? ch.h0f() : (CT)0;
-  CT na[R], nb[R], nh[GRAD ? R : 1];
-  auto fetch = [&](int base) {  // reads at clamped positions
+  CT na[R] = {}, nb[R] = {}, nh[GRAD ? R : 1] = {};
+  auto read = [&](int pos, int r) {
+    na[r] = ch.mult(pos);
+    nb[r] = ch.b_at(ch.t_of(pos));
+    if constexpr (GRAD) nh[r] = ch.hprev_at(pos);
+  };
+  // A row lane past the end of the sequence reads nothing, the one at the end at clamped positions.
+  // (One copy of the reads: a second one for whole tiles costs a short scan more than it saves.)
+  auto fetch = [&](int base) {
+    if (base + step(0) >= L) return;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int pos = min(base + step(r), L - 1);
-      na[r] = ch.mult(pos);
-      nb[r] = ch.b_at(ch.t_of(pos));
-      if constexpr (GRAD) nh[r] = ch.hprev_at(pos);
-    }
+    for (int r = 0; r < R; ++r) read(min(base + step(r), L - 1), r);
   };
   fetch(0);
   int buf = 0;
@@ -135,6 +141,72 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
       if (mval && pos < L) ch.template put<GRAD>(pos, b[r], hp[GRAD ? r : 0]);
       if (GRAD && mval && pos + 1 == L) ch.put_dh0(b[r]);
     }
+  }
+}
+
+// ------------------------------------------------------------------ sequential, one wavefront
+// Sequential, forward, float, unit stride along m.  A wavefront owns 64 consecutive recurrences m of one
+// batch row and walks 16-step blocks.  A block's a and b tiles (16 steps x 64 recurrences) are read
+// with 16-byte loads -- a lane reads 4 recurrences of one step, so one load instruction carries 4
+// steps where a read per recurrence carries one -- and transposed through LDS so that each lane
+// walks its own recurrence; the block's states go back through LDS and leave as 16-byte stores.
+// Reads run kSeqTAhead blocks ahead, at clamped positions (past the end: re-reads of the last step,
+// never used).
+constexpr int kSeqTB = 16, kSeqTAhead = 3;
+typedef float f32x4 __attribute__((ext_vector_type(4)));  // a native vector (HIP's float4 is a struct)
+
+__global__ void __launch_bounds__(64) k_lscan_seqt(const LscanParams P) {
+  __shared__ __align__(16) float sA[kSeqTB][64], sB[kSeqTB][64], sH[kSeqTB][64];
+  const int lane = threadIdx.x;
+  const int64_t b = blockIdx.y, m0 = (int64_t)blockIdx.x * 64;
+  const int L = (int)P.L;
+  const int rl = lane / 16, cl = (lane % 16) * 4;  // the lane's row in a group of 4 steps, its column
+  Chain<float> ch{P, b, m0 + lane};
+  float h = ch.h0();
+  const float *pa = (const float *)P.a.p + b * P.a.s0 + m0 + cl;
+  const float *pb = (const float *)P.b.p + b * P.b.s0 + m0 + cl;
+  float *ph = (float *)P.h.p + b * P.h.s0 + m0 + cl;
+  struct Blk {
+    f32x4 a[kSeqTB / 4], b[kSeqTB / 4];
+  };
+  auto fetch = [&](Blk &k, int pos0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kSeqTB / 4; ++j) {
+      const int64_t t = ch.t_of(min(pos0 + rl + 4 * j, L - 1));
+      k.a[j] = *(const f32x4 *)(pa + t * P.a.s1);
+      k.b[j] = *(const f32x4 *)(pb + t * P.b.s1);
+    }
+  };
+  auto run = [&](const Blk &k, int pos0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kSeqTB / 4; ++j) {
+      *(f32x4 *)&sA[rl + 4 * j][cl] = k.a[j];
+      *(f32x4 *)&sB[rl + 4 * j][cl] = k.b[j];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < kSeqTB; ++r) {
+      h = fmaf(sA[r][lane], h, sB[r][lane]);
+      sH[r][lane] = h;
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < kSeqTB / 4; ++j) {
+      const int pos = pos0 + rl + 4 * j;
+      const f32x4 v = *(const f32x4 *)&sH[rl + 4 * j][cl];
+      if (pos < L) *(f32x4 *)(ph + (int64_t)ch.t_of(pos) * P.h.s1) = v;
+    }
+    wave_lds_sync();  // the next block's tiles reuse the LDS
+  };
+  Blk k[kSeqTAhead];
+  static_for<0, kSeqTAhead>([&](auto icst) { fetch(k[decltype(icst)::value], decltype(icst)::value * kSeqTB); });
+  for (int pos = 0; pos < L; pos += kSeqTAhead * kSeqTB) {
+    // blocks past the end are skipped (their reads, clamped, are never used)
+    static_for<0, kSeqTAhead>([&](auto icst) {
+      constexpr int i = decltype(icst)::value;
+      if (pos + i * kSeqTB < L) run(k[i], pos + i * kSeqTB);
+      fetch(k[i], pos + (i + kSeqTAhead) * kSeqTB);
+    });
   }
 }
 
@@ -240,35 +312,61 @@ __global__ void __launch_bounds__(256) k_lscan_chunk_scan(const LscanParams P) {
 static int64_t walk_groups(const LscanParams &P) { return P.B * ((P.M + kScanMC - 1) / kScanMC); }
 
 // The chunked algorithm walks in one pass (each input read once) where its workgroups fill
-// enough of the GPU, and in three launches (a and b read twice, every chunk in parallel) below:
-// L 4096 float32, forward + adjoint: 256 workgroups 151 + 280 us in one pass, 296 + 426 in three
-// launches; 192: 131 + 241, 209 + 296; 128: 129 + 218, 135 + 210; L 8192, 32: 236 + 413, 67 + 110.
+// enough of the GPU, and in three launches (a and b read twice, every chunk in parallel) below.
+// Forward, forward + adjoint in us, one pass against three launches, L 4096 float32: 192 workgroups
+// 133, 328 against 208, 476; 160 127, 315 against 177, 398; 128 123, 306 against 141, 311; 96 122, 301
+// against 89, 231; L 16384, 64: 473, 1174 against 300, 724.
 static bool chunk_one_pass(const LscanParams &P) { return walk_groups(P) >= 160; }
 
-// Row lanes per workgroup: 8 keep enough reads in flight from one workgroup per CU (256
-// workgroups, forward + adjoint: 4 row lanes 165 + 349 us, 8 151 + 280, 16 164 + 338).  A forward
-// walk with two to four workgroups per CU has enough with 4 and moves fewer rows at a time (L 4096,
-// 512 workgroups: chunked 322 against 332 us, blelloch 317 against 334, sequential 318 against
-// 334; 1,024 workgroups of L 2048: 336 against 325); Hillis-Steele is faster with 8 there too
-// (321 against 326).
+// Row lanes per workgroup.  8 keep enough reads in flight from one workgroup per CU (256 workgroups of
+// L 4096, forward + adjoint: 4 row lanes 165 + 349 us, 8 151 + 280, 16 164 + 338).  Two such
+// workgroups fit a CU (registers; Hillis-Steele: LDS), so from 512 workgroups on, Hillis-Steele past
+// it, 4 row lanes run in one round what 8 run in two (625 workgroups, hillis_steele, L 80 forward
+// 16 -> 11 us), until 1,024 fill two rounds either way (L 2048: 326 us with 8, 340 with 4); short
+// sequences keep 4, whose workgroups hide each other's latencies (forward + adjoint, 1,024
+// workgroups, 8 -> 4: L 80 blelloch 46 -> 39, hillis_steele 45 -> 34; L 400 181 -> 178, 176 -> 169;
+// L 1000 424 -> 443, 433 -> 429).  A sequence of at most 4, 2 or 1 row lanes' steps takes no more
+// than these (sequential, 1,024 workgroups, 8 -> this: L 64 44 -> 26, L 16 39 -> 11).
 template <typename CT, int ALGO, bool GRAD>
 static hipError_t launch_walk(const LscanParams &P, hipStream_t s) {
   const dim3 tiles((unsigned)((P.M + kScanMC - 1) / kScanMC), (unsigned)P.B);
   const int64_t g = walk_groups(P);
-  if constexpr (!GRAD && ALGO != kHs) {
-    if (g >= 512 && g < 1024) {
-      hipLaunchKernelGGL((k_lscan_walk<CT, ALGO, 4, false>), tiles, dim3(4 * kScanMC), 0, s, P);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((k_lscan_walk<CT, ALGO, 8, GRAD>), tiles, dim3(8 * kScanMC), 0, s, P);
+  constexpr int R = scan_rows(ALGO);
+  const bool four = g >= (ALGO == kHs ? 513 : 512) && (P.L <= 512 || g < 1024);
+#define WALK(RL) hipLaunchKernelGGL((k_lscan_walk<CT, ALGO, RL, GRAD>), tiles, dim3(RL * kScanMC), 0, s, P)
+  if (P.L <= R) WALK(1);
+  else if (P.L <= 2 * R) WALK(2);
+  else if (P.L <= 4 * R || four) WALK(4);
+  else WALK(8);
+#undef WALK
   return hipGetLastError();
+}
+
+// The one-wavefront kernel's conditions: unit stride along m, 16-byte aligned rows, M a multiple of
+// 64.  It is taken where a workgroup's barriers cost more than its row lanes hide.  Forward, us,
+// walk -> this: 16 workgroups, L 16 4.1 -> 3.0, L 48 5.0 -> 4.1, L 64 4.5 -> 5.1, L 80 6.4 -> 5.6,
+// L 100 6.2 -> 6.8; 512 workgroups of L 2048 161 -> 154, 1,024 326 -> 308, 256 75 -> 94; 2,048 of
+// L 80 24 -> 21, of L 400 139 -> 131, of L 1000 319 -> 325.
+static bool seqt_ok(const LscanParams &P) {
+  auto ok = [](const KView &v) {
+    return v.s2 == 1 && v.s1 % 4 == 0 && v.s0 % 4 == 0 && ((uintptr_t)v.p % 16) == 0;
+  };
+  const int64_t g = walk_groups(P);
+  return P.M % kScanMC == 0 && ok(P.a) && ok(P.b) && ok(P.h) && 
+         (P.L <= 48 || (P.L > 64 && P.L <= 96) || (g >= 512 && (g <= 1536 || P.L <= 512)));
 }
 
 template <typename CT, bool GRAD>
 static hipError_t launch_lscan_t(const LscanParams &P, int algo, hipStream_t s) {
   switch (algo) {
-    case kSeq: return launch_walk<CT, kSeq, GRAD>(P, s);
+    case kSeq:
+      if constexpr (!GRAD && sizeof(CT) == 4) {
+        if (!P.shift && seqt_ok(P)) {
+          hipLaunchKernelGGL(k_lscan_seqt, dim3((unsigned)(P.M / kScanMC), (unsigned)P.B), dim3(kWave), 0, s, P);
+          return hipGetLastError();
+        }
+      }
+      return launch_walk<CT, kSeq, GRAD>(P, s);
     case kHs: return launch_walk<CT, kHs, GRAD>(P, s);
     case kBl: return launch_walk<CT, kBl, GRAD>(P, s);
   }

@@ -41,8 +41,9 @@ template <typename CT, int ALGO, int RL, int R>
 __device__ __forceinline__ void tile_scan(TileLds<CT, ALGO, RL, R> &X, CT (&a)[R], CT (&b)[R], CT &carry, CT &hin,
                                           int tr, int mi, int &buf) {
   if constexpr (ALGO == kSeq) {
-    // The row lanes take turns: a handover and R dependent updates each.
-    static_assert(RL % 2 == 0, "the last turn's handover is in h[1]");
+    // The row lanes take turns: a handover and R dependent updates each.  (RL is even, or 1: the next
+    // call's first turn writes the half that the last handover of this one is not in.)
+    static_assert(RL == 1 || RL % 2 == 0, "row lanes");
 #pragma unroll
     for (int q = 0; q < RL; ++q) {
       if (q == tr) {
@@ -57,7 +58,7 @@ __device__ __forceinline__ void tile_scan(TileLds<CT, ALGO, RL, R> &X, CT (&a)[R
       }
       lds_barrier();
     }
-    carry = X.h[1][mi];
+    carry = X.h[(RL - 1) & 1][mi];
   } else if constexpr (ALGO == kHs) {
     // At offset o every step k >= o composes with step k - o of the previous pass.  The
     // offsets below RL pair different row lanes (step k - o is in row lane tr - o, or one

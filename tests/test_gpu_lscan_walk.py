@@ -32,11 +32,16 @@ def _ref(a, b, h0, dh, reverse):
 
 
 # (B, L, M): one workgroup; ragged; 160 workgroups and one fewer; 512 and 1,024 (4 and 8 row lanes)
+# ... and the lengths and widths that change the row lanes: 16, 32 and 64 steps (8, 16 and 32 for
+# hillis_steele), 48, 64 and 96 (sequential's one-wavefront forward; 70 columns are not its own), 512
+# steps at 512 and 1,024 workgroups
+SHORT = [(2, L, M) for L in (3, 8, 9, 16, 17, 31, 32, 33, 48, 49, 64, 65, 96, 97) for M in (64, 70)] + [
+    (1, 40, 65600), (4, 80, 8192), (1, 512, 32832), (3, 513, 10944), (1, 130, 98368)]
 SHAPES = [(1, 1, 1), (1, 15, 64), (2, 64, 65), (1, 127, 63), (2, 128, 64), (1, 129, 130), (1, 257, 70),
           (1, 63, 10240), (1, 130, 10177), (1, 66, 10176), (2, 70, 16384), (4, 33, 16384)]
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("shape", SHAPES + SHORT, ids=str)
 @pytest.mark.parametrize("algo", ALGOS)
 def test_walk_edges(algo, shape):
     B, L, M = shape
