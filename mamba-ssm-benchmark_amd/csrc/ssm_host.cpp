@@ -560,7 +560,7 @@ PYBIND11_MODULE(_ssmhost, m) {
   m.def("lscan_backward", torch::wrap_pybind_function(lscan_backward));
   m.def("cscan_forward", torch::wrap_pybind_function(cscan_forward));
   m.def("cscan_backward", torch::wrap_pybind_function(cscan_backward));
-  m.def("abi_version", &ssm_abi_version);
+  m.attr("ABI_VERSION") = SSM_ABI_VERSION;  // of the header the argument structs above were compiled from
   py::class_<DecodePlan>(m, "DecodePlan")
       .def(py::init<const std::vector<std::pair<std::vector<Tensor>, double>> &, Tensor, int64_t, int64_t, int64_t, int64_t,
                     int64_t, int64_t, int, double>())

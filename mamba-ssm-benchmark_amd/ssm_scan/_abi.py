@@ -228,8 +228,9 @@ def host():
         except ImportError as e:
             raise RuntimeError("ssm_scan/_ssmhost.so is missing or does not load: build it with "
                                "__graft_entry__.build() (make -C mamba-ssm-benchmark_amd/csrc)") from e
-        if _ssmhost.abi_version() != ABI_VERSION:
-            raise RuntimeError(f"_ssmhost ABI version {_ssmhost.abi_version()} != expected {ABI_VERSION}")
+        built = getattr(_ssmhost, "ABI_VERSION", None)   # compiled in: lib() has checked the library's own
+        if built != ABI_VERSION:
+            raise RuntimeError(f"_ssmhost was built for ABI version {built}, expected {ABI_VERSION}")
         _host = _ssmhost
     return _host
 

@@ -46,7 +46,7 @@ def test_ctypes_layout_matches_c_header(tmp_path):
     structs = {"ssm_tensor": _abi.Tensor, "ssm_fwd_args": _abi.FwdArgs, "ssm_bwd_args": _abi.BwdArgs,
                "ssm_step_args": _abi.StepArgs, "ssm_decode_args": _abi.DecodeArgs, "ssm_lscan_args": _abi.LscanArgs,
                "ssm_decode_block": _abi.DecodeBlock, "ssm_decode_stack_args": _abi.DecodeStackArgs,
-               "ssm_lscan_bwd_args": _abi.LscanBwdArgs,
+               "ssm_lscan_bwd_args": _abi.LscanBwdArgs, "ssm_cscan_args": _abi.CscanArgs,
                "ssm_disc_args": _abi.DiscArgs, "ssm_conv_args": _abi.ConvArgs, "ssm_norm_args": _abi.NormArgs}
     lines = ['#include <stdio.h>', '#include <stddef.h>', f'#include "{HEADER}"', "int main(void){"]
     for cname, py in structs.items():
@@ -437,3 +437,16 @@ def test_disc_lane_offsets_validated():
     a.Bm.stride[2] = -1
     with pytest.raises(ValueError, match="inner stride"):
         _abi.check(lib.ssm_disc_check(ctypes.byref(a)), "ssm_disc")
+
+
+def test_binding_built_for_another_abi_is_refused(monkeypatch):
+    """The binding reports the header it was compiled from, not the loaded library's version."""
+    import sys
+    from types import SimpleNamespace
+    assert _abi.host().ABI_VERSION == _abi.ABI_VERSION
+    stale = SimpleNamespace(ABI_VERSION=_abi.ABI_VERSION - 1, abi_version=_abi.lib().ssm_abi_version)
+    monkeypatch.setattr(_abi, "_host", None)
+    monkeypatch.setitem(sys.modules, "ssm_scan._ssmhost", stale)
+    monkeypatch.setattr(ssm_scan, "_ssmhost", stale)
+    with pytest.raises(RuntimeError, match="ABI"):
+        _abi.host()
