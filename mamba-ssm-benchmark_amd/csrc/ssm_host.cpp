@@ -97,6 +97,15 @@ struct Launch {
   void *stream;
   explicit Launch(const Tensor &t)
       : guard(t.device()), stream((void *)c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+  // One launch.  `timer` (a profiling.KernelTimer, or None) records its events right around it: the
+  // operand checks, casts and allocations of the call are outside.
+  template <typename Args>
+  void run(const char *what, int (*fn)(const Args *, void *), const Args &args, const py::object &timer = py::none()) const {
+    const py::object end = timer.is_none() ? timer : timer.attr("begin")(what);
+    const int rc = fn(&args, stream);
+    if (!end.is_none()) end.attr("record")();
+    check(rc, what);
+  }
 };
 
 // ------------------------------------------------------------------ fused scan
@@ -146,7 +155,7 @@ void fill_scan(Args &a, const Tensor &x, const Tensor &delta, const Tensor &A, c
 // (out in the io dtype, last, the tensors scan_backward needs)
 py::tuple scan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, const Tensor &Bm, const Tensor &Cm,
                        const OptTensor &D_, const OptTensor &z_, const OptTensor &bias_, const OptTensor &h0_, int method,
-                       bool softplus, int segments, const OptTensor &proj_, bool a_log, bool need_saved) {
+                       bool softplus, int segments, const OptTensor &proj_, bool a_log, bool need_saved, const py::object &timer) {
   at::ScalarType ct = c10::promoteTypes(x.scalar_type(), at::kFloat), io = at::kFloat;
   const Tensor z = get(z_);
   if (ct == at::kDouble) {
@@ -178,7 +187,7 @@ py::tuple scan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, co
     a.saved = saved.data_ptr();
   }
   const Launch l(x);
-  check(ssm_fwd(&a, l.stream), "ssm_fwd");
+  l.run("ssm_fwd", ssm_fwd, a, timer);
   return py::make_tuple(o, last, py::make_tuple(xs, ds, As, Bs, Cs, out(Dv), out(zs), out(bv), out(h0), out(W), out(saved)));
 }
 
@@ -186,7 +195,7 @@ py::tuple scan_backward(const Tensor &xs, const Tensor &ds, const Tensor &As, co
                         const OptTensor &Dv_, const OptTensor &zs_, const OptTensor &bv_, const OptTensor &h0_,
                         const OptTensor &W_, const Tensor &saved, int method, bool softplus, bool a_log, int segments,
                         const OptTensor &dout_, const OptTensor &dlast_, const OptTensor &dz_, const OptTensor &dB_,
-                        const OptTensor &dC_) {
+                        const OptTensor &dC_, const py::object &timer) {
   const Tensor Dv = get(Dv_), zs = get(zs_), bv = get(bv_), h0 = get(h0_), W = get(W_);
   const at::ScalarType io = xs.scalar_type(), ct = As.scalar_type();
   const Tensor dout = dout_ ? cast(*dout_, io) : at::zeros(xs.sizes(), xs.options());
@@ -209,7 +218,7 @@ py::tuple scan_backward(const Tensor &xs, const Tensor &ds, const Tensor &As, co
   a.workspace = ws.data_ptr();
   a.workspace_bytes = n;
   const Launch l(xs);
-  check(ssm_bwd(&a, l.stream), "ssm_bwd");
+  l.run("ssm_bwd", ssm_bwd, a, timer);
   return py::make_tuple(dx, dd, dA, dB, dC, out(dD), out(dz), out(db), out(dh0));
 }
 
@@ -230,7 +239,7 @@ Tensor conv_forward(const Tensor &x, const Tensor &w, const OptTensor &bias, boo
   a.out = view(o);
   if (state) a.state_in = a.state_out = view(*state);
   const Launch l(x);
-  check(ssm_conv_fwd(&a, l.stream), "ssm_conv_fwd");
+  l.run("ssm_conv_fwd", ssm_conv_fwd, a);
   return o;
 }
 
@@ -246,7 +255,7 @@ py::tuple conv_backward(const Tensor &x, const Tensor &w, const OptTensor &bias_
   a.workspace = ws.data_ptr();
   a.workspace_bytes = n;
   const Launch l(x);
-  check(ssm_conv_bwd(&a, l.stream), "ssm_conv_bwd");
+  l.run("ssm_conv_bwd", ssm_conv_bwd, a);
   return py::make_tuple(dx, dw, out(db));
 }
 
@@ -275,7 +284,7 @@ py::tuple norm_forward(const Tensor &x, const Tensor &weight, double eps) {
   a.out = view(o);
   a.rstd = rstd.data_ptr();
   const Launch l(x);
-  check(ssm_norm_fwd(&a, l.stream), "ssm_norm_fwd");
+  l.run("ssm_norm_fwd", ssm_norm_fwd, a);
   return py::make_tuple(o.view(x.sizes()), x2, w, rstd);
 }
 
@@ -292,7 +301,7 @@ py::tuple norm_backward(const Tensor &x2, const Tensor &w, const Tensor &rstd, c
   a.workspace = ws.data_ptr();
   a.workspace_bytes = n;
   const Launch l(x2);
-  check(ssm_norm_bwd(&a, l.stream), "ssm_norm_bwd");
+  l.run("ssm_norm_bwd", ssm_norm_bwd, a);
   return py::make_tuple(dx.view(dout.sizes()), dw);
 }
 
@@ -307,7 +316,8 @@ void fill_lscan(Args &args, const Tensor &a, int algo, int64_t chunk, bool rever
   args.chunk = chunk;
 }
 
-Tensor lscan_forward(const Tensor &a, const Tensor &b, const OptTensor &h0, int algo, int64_t chunk, bool reverse) {
+Tensor lscan_forward(const Tensor &a, const Tensor &b, const OptTensor &h0, int algo, int64_t chunk, bool reverse,
+                     const py::object &timer) {
   const Tensor h = at::empty(a.sizes(), a.options());
   ssm_lscan_args args;
   fill_lscan(args, a, algo, chunk, reverse);
@@ -320,12 +330,12 @@ Tensor lscan_forward(const Tensor &a, const Tensor &b, const OptTensor &h0, int 
     args.workspace_bytes = n;
   }
   const Launch l(a);
-  check(ssm_lscan(&args, l.stream), "ssm_lscan");
+  l.run("ssm_lscan", ssm_lscan, args, timer);
   return h;
 }
 
 py::tuple lscan_backward(const Tensor &a, const OptTensor &h0_, const Tensor &h, const Tensor &dh, int algo, int64_t chunk,
-                         bool reverse, bool need_dh0) {
+                         bool reverse, bool need_dh0, const py::object &timer) {
   const Tensor h0 = get(h0_);
   const Tensor da = at::empty_like(h), db = at::empty_like(h);
   const Tensor dh0 = h0.defined() && need_dh0 ? at::empty_like(h0) : Tensor();
@@ -341,7 +351,7 @@ py::tuple lscan_backward(const Tensor &a, const OptTensor &h0_, const Tensor &h,
     args.workspace_bytes = n;
   }
   const Launch l(a);
-  check(ssm_lscan_bwd(&args, l.stream), "ssm_lscan_bwd");
+  l.run("ssm_lscan_bwd", ssm_lscan_bwd, args, timer);
   return py::make_tuple(da, db, out(dh0));
 }
 
@@ -377,7 +387,7 @@ ssm_cscan_args cscan_args(const Tensor &x, const Tensor &delta, const Tensor &A,
 
 // (y, last, Bm, Cm, saved)
 py::tuple cscan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, const Tensor &Bm_, const Tensor &Cm_,
-                        const OptTensor &h0_, int algo, int method, bool need_saved) {
+                        const OptTensor &h0_, int algo, int method, bool need_saved, const py::object &timer) {
   const Tensor Bm = steps_fit(Bm_), Cm = steps_fit(Cm_), h0 = get(h0_);
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.size(1);
   const Tensor y = at::empty_like(x), last = at::empty({B, D, N}, x.options());
@@ -393,7 +403,7 @@ py::tuple cscan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, c
     ssm_cscan_args a = cscan_args(xb, db, A, Bm, Cm, h0, saved, i, n, algo, method);
     a.y = view(chans(y, 2, i, n));
     a.last = view(chans(last, 1, i, n));
-    check(ssm_cscan_fwd(&a, l.stream), "ssm_cscan_fwd");
+    l.run("ssm_cscan_fwd", ssm_cscan_fwd, a, timer);
   }
   return py::make_tuple(y, last, Bm, Cm, out(saved));
 }
@@ -402,7 +412,7 @@ py::tuple cscan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, c
 // partials (2 x L x NP per 64 / NP channels and batch row) within kCscanWorkspace.
 py::tuple cscan_backward(const Tensor &x, const Tensor &delta, const Tensor &A, const Tensor &Bm, const Tensor &Cm,
                          const OptTensor &h0_, const Tensor &saved, int algo, int method, int64_t d_block,
-                         const OptTensor &dy_, const OptTensor &dlast_) {
+                         const OptTensor &dy_, const OptTensor &dlast_, const py::object &timer) {
   const Tensor h0 = get(h0_), dlast = get(dlast_);
   const Tensor dy = dy_ ? *dy_ : at::zeros_like(x);
   const int64_t B = x.size(0), L = x.size(1), D = x.size(2), N = A.size(1);
@@ -429,7 +439,7 @@ py::tuple cscan_backward(const Tensor &x, const Tensor &delta, const Tensor &A, 
     const Tensor ws = bytes(nb, x);
     a.workspace = ws.data_ptr();
     a.workspace_bytes = nb;
-    check(ssm_cscan_bwd(&a, l.stream), "ssm_cscan_bwd");
+    l.run("ssm_cscan_bwd", ssm_cscan_bwd, a, timer);
     if (!dB.defined()) {
       dB = gB;
       dC = gC;
@@ -541,7 +551,7 @@ struct DecodePlan {
     a.workspace = ws.data_ptr();
     a.workspace_bytes = ws.numel();
     const Launch l(u);
-    check(ssm_decode_stack(&a, l.stream), "ssm_decode_stack");
+    l.run("ssm_decode_stack", ssm_decode_stack, a);
     return logits;
   }
 };

@@ -16,9 +16,8 @@ torch's deterministic mode, kernels/triton_scan.py:298).
 
 import torch
 
-from . import _abi
+from . import _abi, profiling
 from .linear import rocblas, weight_grad
-from .profiling import timed_launch
 
 ZOH, EULER, BILINEAR = 0, 1, 2
 METHODS = {"zoh": ZOH, "euler": EULER, "bilinear": BILINEAR}     # kernels/triton_scan.py:23-24
@@ -70,8 +69,8 @@ def scan_forward(x, delta, A, Bm, Cm, D, z, delta_bias, h0, method, delta_softpl
     scan_backward needs: the tensors as the kernels read them, the saved chunk states and the
     launch settings."""
     segments, a_log, softplus = int(segments or 0), bool(A_is_log), bool(delta_softplus)
-    out, last, tensors = timed_launch("ssm_fwd", _abi.host().scan_forward, x, delta, A, Bm, Cm, D, z, delta_bias, h0,
-                                      method, softplus, segments, delta_proj, a_log, need_saved)
+    out, last, tensors = _abi.host().scan_forward(x, delta, A, Bm, Cm, D, z, delta_bias, h0, method, softplus, segments,
+                                                  delta_proj, a_log, need_saved, profiling.active())
     return out, last, (tensors, (method, softplus, tensors[0].dtype, tensors[2].dtype, a_log, segments))
 
 
@@ -81,8 +80,8 @@ def scan_backward(tensors, settings, dout, dlast, dz=None, dB=None, dC=None):
     Returns (dx, ddelta, dA, dB, dC, dD, dz, ddelta_bias, dh0); with a delta projection,
     ddelta is the gradient of the projected (B, L, D) delta."""
     method, softplus, _, _, a_log, segments = settings
-    return timed_launch("ssm_bwd", _abi.host().scan_backward, *tensors, method, softplus, a_log, segments, dout, dlast,
-                        dz, dB, dC)
+    return _abi.host().scan_backward(*tensors, method, softplus, a_log, segments, dout, dlast, dz, dB, dC,
+                                     profiling.active())
 
 
 def _cast_keep(t, dt):

@@ -1,9 +1,10 @@
 """Optional per-launch timing of the engine's entry points with HIP events.
 
-Inside ``with KernelTimer() as t:`` every C-ABI launch made by this package is bracketed by
-two events recorded on the stream the kernels are enqueued on (torch's current stream),
-so ``t.times_ms()`` gives each entry point's device time per call.  Outside a timer nothing
-is recorded and launches are not touched.
+Inside ``with KernelTimer() as t:`` every launch of a scan, a linear scan or a discretization is
+bracketed by two events recorded on the stream the kernels are enqueued on (torch's current
+stream), right around the C-ABI call: operand checks, casts and allocations come before the first.
+``t.times_ms()`` gives each entry point's device time per launch.  Outside a timer nothing is
+recorded and launches are not touched.
 """
 
 import torch
@@ -26,20 +27,18 @@ class KernelTimer:
         _active = self._prev
         return False
 
+    def begin(self, name):
+        """Records the start of one launch of `name`; returns the event to record at its end."""
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        self.records.setdefault(name, []).append((start, end))
+        start.record()
+        return end
+
     def times_ms(self):
         torch.cuda.synchronize()
         return {k: [s.elapsed_time(e) for s, e in v] for k, v in self.records.items()}
 
 
-def timed_launch(name, fn, *args):
-    """fn(*args), which issues one launch (its result passes through)."""
-    t = _active
-    if t is None:
-        return fn(*args)
-    start = torch.cuda.Event(enable_timing=True)
-    end = torch.cuda.Event(enable_timing=True)
-    start.record()
-    res = fn(*args)
-    end.record()
-    t.records.setdefault(name, []).append((start, end))
-    return res
+def active():
+    """The timer in effect, or None."""
+    return _active

@@ -24,9 +24,8 @@ import ctypes
 
 import torch
 
-from . import _abi, plan
+from . import _abi, plan, profiling
 from .hip_scan import METHODS, FusedSelectiveScanFn, _require_gpu, check_operands
-from .profiling import timed_launch
 
 DISCRETIZATIONS = ("zoh", "euler", "bilinear")      # models/scan.py:36
 SCAN_ELEMENT_BUDGET = plan.SCAN_ELEMENT_BUDGET       # models/scan.py:182
@@ -54,7 +53,11 @@ def _ct(*ts):
 def _launch(name, fn, args, dev):
     with _abi.on_device(dev):
         stream = _abi.stream_handle(dev)
-        rc = timed_launch(name, fn, ctypes.byref(args), stream)
+        timer = profiling.active()
+        end = None if timer is None else timer.begin(name)
+        rc = fn(ctypes.byref(args), stream)
+        if end is not None:
+            end.record()
     _abi.check(rc, name)
 
 
@@ -137,7 +140,7 @@ class LinearScanFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, h0, algo, chunk, reverse):
         cfg = (algo, int(chunk or 0), bool(reverse))
-        h = timed_launch("ssm_lscan", _abi.host().lscan_forward, a, b, h0, *cfg)
+        h = _abi.host().lscan_forward(a, b, h0, *cfg, profiling.active())
         ctx.save_for_backward(a, h0, h)
         ctx.cfg = cfg
         return h
@@ -145,8 +148,7 @@ class LinearScanFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dh):
         a, h0, h = ctx.saved_tensors
-        da, db, dh0 = timed_launch("ssm_lscan_bwd", _abi.host().lscan_backward, a, h0, h, dh, *ctx.cfg,
-                                   ctx.needs_input_grad[2])
+        da, db, dh0 = _abi.host().lscan_backward(a, h0, h, dh, *ctx.cfg, ctx.needs_input_grad[2], profiling.active())
         return da, db, dh0, None, None, None
 
 
@@ -224,8 +226,8 @@ class SelectiveScanFn(torch.autograd.Function):
         chunk = int(chunk_size or 0)
         if not 0 <= chunk < 1 << 30:
             raise ValueError(f"chunk={chunk} out of range")
-        y, last, Bm, Cm, saved = timed_launch("ssm_cscan_fwd", _abi.host().cscan_forward, x, delta, A, Bm, Cm, h0, algo,
-                                              METHODS[method], any(ctx.needs_input_grad[:6]))
+        y, last, Bm, Cm, saved = _abi.host().cscan_forward(x, delta, A, Bm, Cm, h0, algo, METHODS[method],
+                                                           any(ctx.needs_input_grad[:6]), profiling.active())
         ctx.save_for_backward(x, delta, A, Bm, Cm, h0, saved)
         ctx.set_materialize_grads(False)   # an unused output passes None (no zero fill)
         ctx.cfg = (algo, METHODS[method], int(d_block or 0))
@@ -233,7 +235,7 @@ class SelectiveScanFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, dlast):
-        grads = timed_launch("ssm_cscan_bwd", _abi.host().cscan_backward, *ctx.saved_tensors, *ctx.cfg, dy, dlast)
+        grads = _abi.host().cscan_backward(*ctx.saved_tensors, *ctx.cfg, dy, dlast, profiling.active())
         return (*grads, None, None, None, None)
 
 
