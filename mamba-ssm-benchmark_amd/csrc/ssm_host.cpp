@@ -97,12 +97,17 @@ struct Launch {
   void *stream;
   explicit Launch(const Tensor &t)
       : guard(t.device()), stream((void *)c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
-  // One launch.  `timer` (a profiling.KernelTimer, or None) records its events right around it: the
-  // operand checks, casts and allocations of the call are outside.
+  // One launch, without the GIL: it blocks while the device's queue is full, and other Python threads
+  // run on.  `timer` (a profiling.KernelTimer, or None) records its events right around it: the operand
+  // checks, casts and allocations of the call are outside.
   template <typename Args>
   void run(const char *what, int (*fn)(const Args *, void *), const Args &args, const py::object &timer = py::none()) const {
     const py::object end = timer.is_none() ? timer : timer.attr("begin")(what);
-    const int rc = fn(&args, stream);
+    int rc;
+    {
+      py::gil_scoped_release release;
+      rc = fn(&args, stream);
+    }
     if (!end.is_none()) end.attr("record")();
     check(rc, what);
   }
