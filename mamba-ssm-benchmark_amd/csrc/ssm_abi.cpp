@@ -540,7 +540,7 @@ static int lscan_common(int64_t B, int64_t L, int64_t M, int algo, int dtype, in
 static int64_t lscan_chunk(int64_t L, int64_t chunk) { return chunk ? chunk : ssm_default_chunk(L); }
 
 static int64_t lscan_ws(int64_t B, int64_t L, int64_t M, int algo, int dtype, int64_t chunk) {
-  if (algo != SSM_SCAN_CHUNKED) return 0;
+  if (algo != SSM_SCAN_CHUNKED || lscan_one_pass(B, M)) return 0;
   return align256(3 * B * cdiv(L, lscan_chunk(L, chunk)) * M * state_size(dtype));
 }
 

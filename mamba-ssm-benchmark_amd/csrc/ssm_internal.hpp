@@ -177,8 +177,14 @@ struct LscanParams {
   // Adjoint (hf set): the scan's values are lambda and go to h (= db); hf is the forward scan's
   // states and h0f its initial state; da and dh0 are written with lambda.
   KView hf, h0f, da, dh0;
-  void *ws;           // chunked: 3 x (B, nc, M) state type (P, E, h_in)
+  void *ws;           // chunked in three launches: 3 x (B, nc, M) state type (P, E, h_in)
 };
+
+// Workgroups of a walk (kScanMC recurrences of a batch row each), and whether the chunked algorithm runs as one
+// (ssm_lscan.hip: the figures behind the line); only its three launches use chunks and a workspace.
+constexpr int kScanMC = 64;
+inline int64_t lscan_groups(int64_t B, int64_t M) { return B * ((M + kScanMC - 1) / kScanMC); }
+inline bool lscan_one_pass(int64_t B, int64_t M) { return lscan_groups(B, M) >= 160; }
 
 // Materialized discretization on contiguous (B, L, D, N) tensors.
 struct DiscParams {

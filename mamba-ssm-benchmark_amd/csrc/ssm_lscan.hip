@@ -91,7 +91,6 @@ struct Chain {
 };
 
 // ------------------------------------------------------------------ the tiled walk
-constexpr int kScanMC = 64;   // recurrences per workgroup
 // Steps per row lane and tile (Hillis-Steele keeps every step of a tile in LDS twice).
 constexpr int scan_rows(int algo) { return algo == kHs ? 8 : 16; }
 
@@ -309,15 +308,6 @@ __global__ void __launch_bounds__(256) k_lscan_chunk_scan(const LscanParams P) {
   chunk_walk<CT, false, GRAD>(P, ch, p0, p1, h, prod);
 }
 
-static int64_t walk_groups(const LscanParams &P) { return P.B * ((P.M + kScanMC - 1) / kScanMC); }
-
-// The chunked algorithm walks in one pass (each input read once) where its workgroups fill
-// enough of the GPU, and in three launches (a and b read twice, every chunk in parallel) below.
-// Forward, forward + adjoint in us, one pass against three launches, L 4096 float32: 192 workgroups
-// 133, 328 against 208, 476; 160 127, 315 against 177, 398; 128 123, 306 against 141, 311; 96 122, 301
-// against 89, 231; L 16384, 64: 473, 1174 against 300, 724.
-static bool chunk_one_pass(const LscanParams &P) { return walk_groups(P) >= 160; }
-
 // Row lanes per workgroup.  8 keep enough reads in flight from one workgroup per CU (256 workgroups of
 // L 4096, forward + adjoint: 4 row lanes 165 + 349 us, 8 151 + 280, 16 164 + 338).  Two such
 // workgroups fit a CU (registers; Hillis-Steele: LDS), so from 512 workgroups on, Hillis-Steele past
@@ -330,7 +320,7 @@ static bool chunk_one_pass(const LscanParams &P) { return walk_groups(P) >= 160;
 template <typename CT, int ALGO, bool GRAD>
 static hipError_t launch_walk(const LscanParams &P, hipStream_t s) {
   const dim3 tiles((unsigned)((P.M + kScanMC - 1) / kScanMC), (unsigned)P.B);
-  const int64_t g = walk_groups(P);
+  const int64_t g = lscan_groups(P.B, P.M);
   constexpr int R = scan_rows(ALGO);
   const bool four = g >= (ALGO == kHs ? 513 : 512) && (P.L <= 512 || g < 1024);
 #define WALK(RL) hipLaunchKernelGGL((k_lscan_walk<CT, ALGO, RL, GRAD>), tiles, dim3(RL * kScanMC), 0, s, P)
@@ -351,7 +341,7 @@ static bool seqt_ok(const LscanParams &P) {
   auto ok = [](const KView &v) {
     return v.s2 == 1 && v.s1 % 4 == 0 && v.s0 % 4 == 0 && ((uintptr_t)v.p % 16) == 0;
   };
-  const int64_t g = walk_groups(P);
+  const int64_t g = lscan_groups(P.B, P.M);
   return P.M % kScanMC == 0 && ok(P.a) && ok(P.b) && ok(P.h) && 
          (P.L <= 48 || (P.L > 64 && P.L <= 96) || (g >= 512 && (g <= 1536 || P.L <= 512)));
 }
@@ -370,7 +360,12 @@ static hipError_t launch_lscan_t(const LscanParams &P, int algo, hipStream_t s) 
     case kHs: return launch_walk<CT, kHs, GRAD>(P, s);
     case kBl: return launch_walk<CT, kBl, GRAD>(P, s);
   }
-  if (chunk_one_pass(P)) return launch_walk<CT, kChunk, GRAD>(P, s);
+  // In one pass (each input read once) where its workgroups fill enough of the GPU, in three launches (a
+  // and b read twice, every chunk in parallel) below.  Forward, forward + adjoint in us, one pass
+  // against three launches, L 4096 float32: 192 workgroups 133, 328 against 208, 476; 160 127, 315
+  // against 177, 398; 128 123, 306 against 141, 311; 96 122, 301 against 89, 231; L 16384, 64: 473,
+  // 1174 against 300, 724.
+  if (lscan_one_pass(P.B, P.M)) return launch_walk<CT, kChunk, GRAD>(P, s);
   const int64_t n = P.B * P.nc * P.M, chains = P.B * P.M;
   hipLaunchKernelGGL((k_lscan_chunk_reduce<CT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, P);
   hipLaunchKernelGGL((k_lscan_chunk_carry<CT>), dim3((unsigned)((chains + 255) / 256)), dim3(256), 0, s, P);

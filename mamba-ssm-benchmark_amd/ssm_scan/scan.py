@@ -188,7 +188,12 @@ def scan_blelloch(a, b, h0=None):
 
 
 def scan_chunked(a, b, h0=None, chunk_size=None):
-    """Two-level scan with chunk size C = chunk_size or default_chunk(L) (models/scan.py:142-165)."""
+    """Two-level scan (models/scan.py:142-165).
+
+    Below 160 groups of 64 recurrences the chunks of C = chunk_size or default_chunk(L) steps are spread
+    over the GPU (three launches; the workspace holds three values per chunk and recurrence).  From
+    there on one launch walks every recurrence in chunks of 16 steps and chunk_size changes
+    nothing.  The result is the same to rounding either way."""
     return _scan("chunked", a, b, h0, chunk_size)
 
 
@@ -256,6 +261,8 @@ def selective_scan(x, delta, A, Bm, Cm, h0=None, method="zoh", scan="chunked",
 
     scan = 'reference' | 'sequential' | 'hillis_steele' | 'blelloch' | 'chunked'
            | 'triton' (the fused engine) | 'auto' (fused when N is a power of two, else chunked)
+    d_block: channels per launch of the backward of the four named algorithms (bounds its workspace);
+    chunk_size is accepted for the reference's signature and changes nothing (SelectiveScanFn).
     Computes in promote(dtype, float32); y is returned in x's dtype, h_last in the compute
     dtype.  KeyError for an unknown scan, ValueError for an unknown method."""
     _require_gpu(x, delta, A, Bm, Cm, h0)

@@ -450,3 +450,16 @@ def test_binding_built_for_another_abi_is_refused(monkeypatch):
     monkeypatch.setattr(ssm_scan, "_ssmhost", stale)
     with pytest.raises(RuntimeError, match="ABI"):
         _abi.host()
+
+
+@pytest.mark.parametrize("width,one_pass", [(159 * 64, False), (159 * 64 + 1, True)])
+def test_linear_scan_workspace_only_for_chunks(width, one_pass):
+    """From 160 workgroups of 64 recurrences on the chunked scan runs in one pass and takes no workspace."""
+    t = torch.zeros(1, 1, 1)
+    lib = _abi.lib()
+    for args, query, names in ((_abi.LscanArgs(), lib.ssm_lscan_workspace_bytes, ("a", "b", "h")),
+                               (_abi.LscanBwdArgs(), lib.ssm_lscan_bwd_workspace_bytes, ("a", "h", "dh", "da", "db"))):
+        args.batch, args.seqlen, args.width, args.algo, args.dtype, args.chunk = 1, 64, width, 4, 0, 4
+        for name in names:
+            setattr(args, name, _abi.view(t))
+        assert query(ctypes.byref(args)) == (0 if one_pass else -(-3 * 16 * width * 4 // 256) * 256)

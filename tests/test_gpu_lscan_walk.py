@@ -70,3 +70,18 @@ def test_walk_strided_and_float64(algo):
     grads = torch.autograd.grad(h, leaves, dh)
     for got, ref in zip((h.detach(), *grads), _ref(a, b, None, dh, False)):
         torch.testing.assert_close(got, ref, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("M", [159 * 64, 159 * 64 + 1])     # three launches and one pass
+@pytest.mark.parametrize("chunk", [1, 7, 300])
+def test_chunk_sizes_on_both_sides_of_the_one_pass_rule(M, chunk):
+    g = torch.Generator(device="cuda").manual_seed(chunk)
+    a = torch.rand(1, 67, M, generator=g, device="cuda") * 0.5 + 0.5
+    b, dh = (torch.randn(1, 67, M, generator=g, device="cuda") for _ in range(2))
+    h0 = torch.randn(1, M, generator=g, device="cuda")
+    leaves = [t.detach().requires_grad_() for t in (a, b, h0)]
+    h = S.scan_chunked(*leaves, chunk_size=chunk)
+    refs = _ref(a, b, h0, dh, False)
+    da_atol = max(1e-5, 16 * 2.0 ** -24 * refs[0].abs().max().item() * refs[2].abs().max().item())  # as above
+    for name, got, ref in zip(("h", "da", "db", "dh0"), (h.detach(), *torch.autograd.grad(h, leaves, dh)), refs):
+        close(got, ref, name=name, **({"atol": da_atol} if name == "da" else {}))
