@@ -313,7 +313,8 @@ typedef struct ssm_cscan_args {
   ssm_tensor dA;           /* backward: (D,N) */
   ssm_tensor dBm, dCm;     /* backward: (B,L,N) */
   ssm_tensor dh0;          /* backward: (B,D,N) optional */
-  void *workspace;         /* backward: ssm_cscan_workspace_bytes() */
+  void *workspace;         /* backward: ssm_cscan_workspace_bytes(); forward:
+                              ssm_cscan_fwd_workspace_bytes(), or less: time is then not split */
   int64_t workspace_bytes;
 } ssm_cscan_args;
 
@@ -400,7 +401,8 @@ int64_t ssm_fwd_workspace_bytes(const ssm_fwd_args *args);
 int64_t ssm_bwd_workspace_bytes(const ssm_bwd_args *args);
 int64_t ssm_lscan_workspace_bytes(const ssm_lscan_args *args);
 int64_t ssm_lscan_bwd_workspace_bytes(const ssm_lscan_bwd_args *args);
-int64_t ssm_cscan_workspace_bytes(const ssm_cscan_args *args);
+int64_t ssm_cscan_fwd_workspace_bytes(const ssm_cscan_args *args);
+int64_t ssm_cscan_workspace_bytes(const ssm_cscan_args *args);   /* backward */
 int64_t ssm_disc_workspace_bytes(const ssm_disc_args *args);
 int64_t ssm_conv_workspace_bytes(const ssm_conv_args *args);
 int64_t ssm_norm_workspace_bytes(const ssm_norm_args *args);

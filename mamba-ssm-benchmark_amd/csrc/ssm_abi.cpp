@@ -759,6 +759,21 @@ int ssm_cscan_check(const ssm_cscan_args *a) {
   return ok();
 }
 
+// The chunked algorithm's time segments: as many as bring the launch to one workgroup per CU, of at least
+// kCscSegTiles time tiles, at most kCscMaxSeg (whose maps a walk folds one by one).  Forward, forward +
+// backward of a replayed graph in us, N 16 float32, whole -> segments: L 1024 D 16 19, 61 -> 13, 32,
+// D 512 20, 72 -> 20, 61; L 16384 D 16 255, 836 -> 21, 57, D 512 272, 963 -> 214, 690.  Shorter
+// sequences stay whole: L 512 D 64 11, 36 -> 13, 32.  (Materialized, L 65536 D 16 took 1.2 and 2.5 ms:
+// whole it takes 1.0 and 3.4 ms, in segments 0.07 and 0.16.)
+constexpr int64_t kCscGroups = 256, kCscSegTiles = 4, kCscMinTiles = 16, kCscMaxSeg = 64;
+static void csc_segments(const ssm_cscan_args *a, CscParams &p) {
+  const int64_t tiles = cdiv(a->seqlen, csc_tile(a->algo, a->dtype == SSM_F64)), groups = a->batch * p.ntiles;
+  int64_t n = 1;
+  if (a->algo == SSM_SCAN_CHUNKED && tiles >= kCscMinTiles) n = std::min({kCscGroups / groups, tiles / kCscSegTiles, kCscMaxSeg});
+  p.seg_tiles = (int)cdiv(tiles, std::max<int64_t>(n, 1));
+  p.nseg = (int)cdiv(tiles, p.seg_tiles);
+}
+
 static CscParams csc_params(const ssm_cscan_args *a) {
   CscParams p;
   memset(&p, 0, sizeof(p));
@@ -768,24 +783,40 @@ static CscParams csc_params(const ssm_cscan_args *a) {
   p.y = kv(a->y); p.last = kv(a->last); p.saved = kv(a->saved);
   p.dy = kv(a->dy); p.dlast = kv(a->dlast); p.dx = kv(a->dx); p.ddelta = kv(a->ddelta);
   p.dA = kv(a->dA); p.dB = kv(a->dBm); p.dC = kv(a->dCm); p.dh0 = kv(a->dh0);
+  csc_segments(a, p);
   return p;
 }
 
+// Workspace: the segments' maps, then (backward) the dB / dC partials and the dA partials.
+static int64_t csc_ws_seg(const CscParams &p, int dtype) {
+  return p.nseg > 1 ? align256(2 * p.B * p.nseg * p.D * p.N * state_size(dtype)) : 0;
+}
 static int64_t csc_ws_bc(const ssm_cscan_args *a, const CscParams &p) {
   return align256(a->batch * p.ntiles * a->seqlen * 2 * padded_n(a->dstate) * state_size(a->dtype));
 }
 
+int64_t ssm_cscan_fwd_workspace_bytes(const ssm_cscan_args *a) {
+  if (ssm_cscan_check(a)) return -1;
+  return csc_ws_seg(csc_params(a), a->dtype);
+}
+
 int64_t ssm_cscan_workspace_bytes(const ssm_cscan_args *a) {
   if (ssm_cscan_check(a)) return -1;
-  return csc_ws_bc(a, csc_params(a)) + align256(a->batch * a->dim * a->dstate * 8);
+  const CscParams p = csc_params(a);
+  return csc_ws_seg(p, a->dtype) + csc_ws_bc(a, p) + align256(p.B * p.nseg * p.D * p.N * 8);
 }
 
 int ssm_cscan_fwd(const ssm_cscan_args *a, void *stream) {
   int rc = ssm_cscan_check(a);
   if (rc) return rc;
   REQUIRE(a->y, "y");
-  const hipError_t e = launch_csc(csc_params(a), a->algo, a->dtype, a->method, padded_n(a->dstate), false,
-                                  (hipStream_t)stream);
+  CscParams p = csc_params(a);
+  if (!a->workspace || a->workspace_bytes < csc_ws_seg(p, a->dtype)) {  // one segment needs none
+    p.seg_tiles *= p.nseg;
+    p.nseg = 1;
+  }
+  p.ws_seg = a->workspace;
+  const hipError_t e = launch_csc(p, a->algo, a->dtype, a->method, padded_n(a->dstate), false, (hipStream_t)stream);
   return e == hipSuccess ? ok() : hip_fail(e, "ssm_cscan_fwd");
 }
 
@@ -802,11 +833,12 @@ int ssm_cscan_bwd(const ssm_cscan_args *a, void *stream) {
   if (has(a->dh0) && !has(a->h0)) return fail(SSM_EINVAL, "dh0 given without h0");
   if ((rc = csc_offsets(a->dy, a->dim, state_size(a->dtype), "dy"))) return rc;
   CscParams p = csc_params(a);
-  const int64_t bc = csc_ws_bc(a, p), need = bc + align256(a->batch * a->dim * a->dstate * 8);
+  const int64_t seg = csc_ws_seg(p, a->dtype), bc = csc_ws_bc(a, p), need = ssm_cscan_workspace_bytes(a);
   if (!a->workspace || a->workspace_bytes < need)
     return fail(SSM_ESPACE, "workspace of %lld bytes required", (long long)need);
-  p.ws_bc = a->workspace;
-  p.ws_dA = (char *)a->workspace + bc;
+  p.ws_seg = a->workspace;
+  p.ws_bc = (char *)a->workspace + seg;
+  p.ws_dA = (char *)a->workspace + seg + bc;
   const hipError_t e = launch_csc(p, a->algo, a->dtype, a->method, padded_n(a->dstate), true, (hipStream_t)stream);
   return e == hipSuccess ? ok() : hip_fail(e, "ssm_cscan_bwd");
 }

@@ -3,7 +3,7 @@
 // contracts, where the reference materializes a, b, h, their gradients and the adjoint.
 //
 // A workgroup owns 64 / NP channels x NP states (one recurrence per lane) of one batch row and walks
-// time in tiles of RL row lanes (wavefronts) x R steps.  Forward: a tile's x, delta, B, C are read
+// time (with the chunked algorithm, few workgroups and a long sequence: one segment of it) in tiles of RL row lanes (wavefronts) x R steps.  Forward: a tile's x, delta, B, C are read
 // while the previous tile is scanned, a and b are formed in registers as k_disc_fwd forms them, and
 // y = sum_n C h is summed over the state lanes before it is stored.  It saves the state entering
 // every tile.  Backward, from the last tile to the first: the tile's states are recomputed from the
@@ -14,6 +14,7 @@
 //   dBm, dCm     sums over the workgroup's channels inside the wavefront; one partial per tile of
 //                channels, which k_csc_fin adds in float64, in a fixed order
 //   dA           float64 running sums of 4-step float sums per lane, one partial per batch row
+//                (and time segment)
 //   dh0          the mu left at the first step
 // All sums run in a fixed order, so results are bitwise reproducible.
 //
@@ -230,7 +231,103 @@ __device__ __forceinline__ CT finite_decay(CT A) {
   return A < lim ? lim : A;
 }
 
-template <typename CT, int NP, int METHOD, int ALGO>
+// ------------------------------------------------------------------ time segments
+// The chunked algorithm splits a long sequence over workgroups where its recurrences alone leave the GPU
+// idle: k_csc_sum forms every segment's affine map (its decay product P and its end value E from
+// zero), and each segment's walk first folds the maps of the segments before it.  In a segment a
+// wavefront takes a contiguous eighth, without exchanges until the end.  BWD: the adjoint's map, against
+// time (mu <- a (C dy + mu)).
+template <typename CT, int NP, int METHOD, bool BWD>
+__global__ void __launch_bounds__((cs_rl<CT, kChunk>() * kWave)) k_csc_sum(const CscParams p) {
+  constexpr int RL = cs_rl<CT, kChunk>(), R = cs_rows<CT, kChunk>(), CW = kWave / NP;
+  __shared__ __align__(16) StageLds<CT, R, NP, false> stage[RL];
+  __shared__ CT sP[RL][kWave], sE[RL][kWave];
+  const int lane = threadIdx.x % kWave, tr = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  StageLds<CT, R, NP, false> &S = stage[tr];
+  const int c = lane / NP, n = lane % NP, d0 = blockIdx.x * CW, d = d0 + c;
+  const int64_t b = blockIdx.y;
+  const int L = (int)p.L, D = (int)p.D, N = (int)p.N;
+  const bool valid = d < D && n < N;
+  const AConst<CT> ac = make_aconst(valid ? finite_decay(vload<CT>(p.A, d * p.A.s0 + n * p.A.s1)) : (CT)-1);
+  const int cr = valid ? c : CW, nr = valid ? n : NP;
+  const TileIn<CT, R, CW> iu(BWD ? p.dy : p.x, b, d0, D, 1, lane), id(p.dt, b, d0, D, 1, lane);
+  const TileIn<CT, R, NP> iV(BWD ? p.Cm : p.Bm, b, 0, N, 1, lane);
+  const int seg = (int)blockIdx.z + (BWD ? 1 : 0);  // nothing follows the last segment, or the adjoint's first
+  const int w0 = (seg * p.seg_tiles * RL + tr * p.seg_tiles) * R, w1 = min(w0 + p.seg_tiles * R, L);
+  CT nu[iu.E], nd[id.E], nV[iV.E];
+  auto fetch = [&](int k) {
+    const int t0 = w0 + k * R, nv = L - t0;
+    iu.load(nu, t0, nv, lane);
+    id.load(nd, t0, nv, lane);
+    iV.load(nV, t0, nv, lane);
+  };
+  const int nb = w0 < w1 ? (w1 - w0 + R - 1) / R : 0;  // the same for the whole wavefront
+  CT P = 1, E = 0;
+  S.clear_pad(lane);
+  if (nb > 0) fetch(BWD ? nb - 1 : 0);
+  for (int k = 0; k < nb; ++k) {
+    iu.stage(S.x, nu, lane);
+    id.stage(S.dt, nd, lane);
+    iV.stage(S.B, nV, lane);
+    wave_lds_sync();
+    if (k + 1 < nb) fetch(BWD ? nb - 2 - k : k + 1);
+    CT dt[R], u[R], V[R];
+    lds_row(&S.dt[cr][0], dt);
+    lds_row(&S.x[cr][0], u);
+    lds_row(&S.B[nr][0], V);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {  // a zero step is the identity
+      const int r = BWD ? R - 1 - q : q;
+      CT a, coef;
+      disc<METHOD>(dt[r], ac, a, coef);
+      if constexpr (BWD) E = a * fma(V[r], u[r], E);
+      else E = fma(a, E, bcoef<METHOD>(dt[r], coef) * (V[r] * u[r]));
+      P *= a;
+    }
+    wave_lds_sync();
+  }
+  sP[tr][lane] = P;
+  sE[tr][lane] = E;
+  lds_barrier();
+  if (tr == 0 && valid) {
+    P = 1;
+    E = 0;
+#pragma unroll
+    for (int q = 0; q < RL; ++q) {
+      const int k = BWD ? RL - 1 - q : q;
+      E = fma(sP[k][lane], E, sE[k][lane]);
+      P *= sP[k][lane];
+    }
+    CT *const ws = (CT *)p.ws_seg;
+    const int64_t o = ((b * p.nseg + seg) * p.D + d) * p.N + n;
+    ws[o] = P;
+    ws[p.B * p.nseg * p.D * p.N + o] = E;
+  }
+}
+
+// v through the maps of `count` segments, the first at s0 and each following `dir` further; 8 are read
+// at a time (clamped to the last), the same folds in every wavefront of a workgroup.
+template <typename CT>
+__device__ __forceinline__ CT seg_fold(const CscParams &p, int64_t b, int d, int n, int s0, int dir, int count, CT v) {
+  const int64_t plane = p.D * p.N, half = p.B * p.nseg * plane;
+  const CT *const ws = (const CT *)p.ws_seg + b * p.nseg * plane + (int64_t)d * p.N + n;
+  for (int k = 0; k < count; k += 8) {
+    CT P[8], E[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int64_t o = (s0 + dir * min(k + j, count - 1)) * plane;
+      P[j] = ws[o];
+      E[j] = ws[half + o];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k + j < count) v = fma(P[j], v, E[j]);
+  }
+  return v;
+}
+
+// ------------------------------------------------------------------ the walks
+template <typename CT, int NP, int METHOD, int ALGO, bool SEG>
 __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const CscParams p) {
   constexpr int RL = cs_rl<CT, ALGO>(), R = cs_rows<CT, ALGO>(), T = RL * R, CW = kWave / NP;
   constexpr int ST = ALGO == kHs ? RL : 1;  // steps between a row lane's consecutive ones
@@ -255,12 +352,15 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
     iB.load(nB, t0, nv, lane);
     iC.load(nC, t0, nv, lane);
   };
-  fetch(0);
+  const int seg = SEG ? (int)blockIdx.z : 0, first = SEG ? seg * p.seg_tiles : 0;
+  const int end = SEG ? min(L, (first + p.seg_tiles) * T) : L;
+  fetch(first * T);
   S.clear_pad(lane);
-  int buf = 0, i = 0;
+  if (SEG && valid) carry = seg_fold<CT>(p, b, d, n, 0, 1, seg, carry);
+  int buf = 0, i = first;
   const int yi = state_index<NP, R>(lane);
   const bool yown = state_owner<NP, R>(lane) && d < D;
-  for (int base = 0; base < L; base += T, ++i) {
+  for (int base = first * T; base < end; base += T, ++i) {
     if (p.saved.p && tr == 0 && valid)
       ((CT *)p.saved.p)[b * p.saved.s0 + i * p.saved.s1 + d * p.saved.s2 + n] = carry;
     ix.stage(S.x, nx, lane);
@@ -268,7 +368,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
     iB.stage(S.B, nB, lane);
     iC.stage(S.C, nC, lane);
     wave_lds_sync();
-    if (base + T < L) fetch(base + T);
+    if (base + T < end) fetch(base + T);
     CT a[R], h[R], y[R], x[R], dt[R], Bv[R];
     lds_row(&S.dt[cr][0], dt);
     lds_row(&S.x[cr][0], x);
@@ -292,10 +392,10 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_fwd(const C
     }
     wave_lds_sync();
   }
-  if (p.last.p && tr == 0 && valid) vstore<CT>(p.last, b * p.last.s0 + d * p.last.s1 + n * p.last.s2, carry);
+  if (p.last.p && end == L && tr == 0 && valid) vstore<CT>(p.last, b * p.last.s0 + d * p.last.s1 + n * p.last.s2, carry);
 }
 
-template <typename CT, int NP, int METHOD, int ALGO>
+template <typename CT, int NP, int METHOD, int ALGO, bool SEG>
 __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const CscParams p) {
   constexpr int RL = cs_rl<CT, ALGO>(), R = cs_rows<CT, ALGO>(), T = RL * R, CW = kWave / NP, V = 2 * R;
   constexpr int ST = ALGO == kHs ? RL : 1;
@@ -325,15 +425,17 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
     iC.load(nC, t0, nv, lane);
     if (valid) nh = ((const CT *)p.saved.p)[b * p.saved.s0 + i * p.saved.s1 + d * p.saved.s2 + n];
   };
-  const int nt = (L + T - 1) / T;
+  const int seg = SEG ? (int)blockIdx.z : 0, first = SEG ? seg * p.seg_tiles : 0;
+  const int all = (L + T - 1) / T, nt = SEG ? min(all, first + p.seg_tiles) : all;  // tiles first .. nt - 1
   fetch(nt - 1);
   S.clear_pad(lane);
+  if (SEG && valid) mu = seg_fold<CT>(p, b, d, n, p.nseg - 1, -1, p.nseg - 1 - seg, mu);
   int buf = 0;
   double gA = 0;
   const int oi = state_index<NP, V>(lane), wi = chan_index<NP, V>(lane);
   const bool own = state_owner<NP, V>(lane) && d < D;
   CT *const ws = (CT *)p.ws_bc + (b * p.ntiles + tile) * p.L * 2 * NP;  // (L, {B, C}, NP) partials
-  for (int i = nt - 1; i >= 0; --i) {
+  for (int i = nt - 1; i >= first; --i) {
     const int base = i * T;
     CT hc = nh;  // the state entering the tile
     const CT hc0 = hc;
@@ -343,7 +445,7 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
     iB.stage(S.B, nB, lane);
     iC.stage(S.C, nC, lane);
     wave_lds_sync();
-    if (i > 0) fetch(i - 1);
+    if (i > first) fetch(i - 1);
     CT a[R], a0[R], coef[R], h[R], dt[R], x[R], Bv[R], dy[R], g[R];
     lds_row(&S.dt[cr][0], dt);
     lds_row(&S.x[cr][0], x);
@@ -432,39 +534,45 @@ __global__ void __launch_bounds__((cs_rl<CT, ALGO>() * kWave)) k_csc_bwd(const C
     double s = 0;
 #pragma unroll
     for (int q = 0; q < RL; ++q) s += red[q][lane];
-    ((double *)p.ws_dA)[(b * p.D + d) * p.N + n] = s;
-    if (p.dh0.p) vstore<CT>(p.dh0, b * p.dh0.s0 + d * p.dh0.s1 + n * p.dh0.s2, mu);
+    ((double *)p.ws_dA)[((SEG ? b * p.nseg + seg : b) * p.D + d) * p.N + n] = s;
+    if (p.dh0.p && seg == 0) vstore<CT>(p.dh0, b * p.dh0.s0 + d * p.dh0.s1 + n * p.dh0.s2, mu);
   }
 }
 
-template <typename CT, int NP, int METHOD, int ALGO>
+template <typename CT, int NP, int METHOD, int ALGO, bool SEG>
 static hipError_t csc_t(const CscParams &p, bool bwd, hipStream_t s) {
   constexpr int CW = kWave / NP;
-  const dim3 grid((unsigned)((p.D + CW - 1) / CW), (unsigned)p.B);
-  if (bwd) hipLaunchKernelGGL((k_csc_bwd<CT, NP, METHOD, ALGO>), grid, dim3(cs_rl<CT, ALGO>() * kWave), 0, s, p);
-  else hipLaunchKernelGGL((k_csc_fwd<CT, NP, METHOD, ALGO>), grid, dim3(cs_rl<CT, ALGO>() * kWave), 0, s, p);
+  const unsigned tiles = (unsigned)((p.D + CW - 1) / CW), threads = cs_rl<CT, ALGO>() * kWave;
+  if constexpr (SEG) {
+    const dim3 g(tiles, (unsigned)p.B, (unsigned)p.nseg - 1);
+    if (bwd) hipLaunchKernelGGL((k_csc_sum<CT, NP, METHOD, true>), g, dim3(threads), 0, s, p);
+    else hipLaunchKernelGGL((k_csc_sum<CT, NP, METHOD, false>), g, dim3(threads), 0, s, p);
+  }
+  const dim3 grid(tiles, (unsigned)p.B, (unsigned)p.nseg);
+  if (bwd) hipLaunchKernelGGL((k_csc_bwd<CT, NP, METHOD, ALGO, SEG>), grid, dim3(threads), 0, s, p);
+  else hipLaunchKernelGGL((k_csc_fwd<CT, NP, METHOD, ALGO, SEG>), grid, dim3(threads), 0, s, p);
   return hipGetLastError();
 }
 
-template <typename CT, int NP, int ALGO>
+template <typename CT, int NP, int ALGO, bool SEG>
 static hipError_t csc_m(const CscParams &p, int method, bool bwd, hipStream_t s) {
-  return method == 0 ? csc_t<CT, NP, 0, ALGO>(p, bwd, s) : method == 1 ? csc_t<CT, NP, 1, ALGO>(p, bwd, s)
-                                                                       : csc_t<CT, NP, 2, ALGO>(p, bwd, s);
+  return method == 0 ? csc_t<CT, NP, 0, ALGO, SEG>(p, bwd, s) : method == 1 ? csc_t<CT, NP, 1, ALGO, SEG>(p, bwd, s)
+                                                                       : csc_t<CT, NP, 2, ALGO, SEG>(p, bwd, s);
 }
 
-template <typename CT, int ALGO>
+template <typename CT, int ALGO, bool SEG>
 static hipError_t csc_n(const CscParams &p, int method, int np, bool bwd, hipStream_t s) {
   switch (np) {
-    case 8: return csc_m<CT, 8, ALGO>(p, method, bwd, s);
-    case 16: return csc_m<CT, 16, ALGO>(p, method, bwd, s);
-    case 32: return csc_m<CT, 32, ALGO>(p, method, bwd, s);
-    default: return csc_m<CT, 64, ALGO>(p, method, bwd, s);
+    case 8: return csc_m<CT, 8, ALGO, SEG>(p, method, bwd, s);
+    case 16: return csc_m<CT, 16, ALGO, SEG>(p, method, bwd, s);
+    case 32: return csc_m<CT, 32, ALGO, SEG>(p, method, bwd, s);
+    default: return csc_m<CT, 64, ALGO, SEG>(p, method, bwd, s);
   }
 }
 
-template <int ALGO>
+template <int ALGO, bool SEG>
 hipError_t launch_csc_algo(const CscParams &p, int dtype, int method, int np, bool bwd, hipStream_t s) {
-  return dtype == 3 ? csc_n<double, ALGO>(p, method, np, bwd, s) : csc_n<float, ALGO>(p, method, np, bwd, s);
+  return dtype == 3 ? csc_n<double, ALGO, SEG>(p, method, np, bwd, s) : csc_n<float, ALGO, SEG>(p, method, np, bwd, s);
 }
 
 }  // namespace ssm

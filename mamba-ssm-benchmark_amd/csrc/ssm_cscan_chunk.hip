@@ -4,12 +4,13 @@
 
 namespace ssm {
 
-template hipError_t launch_csc_algo<kChunk>(const CscParams &, int, int, int, bool, hipStream_t);
-extern template hipError_t launch_csc_algo<kSeq>(const CscParams &, int, int, int, bool, hipStream_t);
-extern template hipError_t launch_csc_algo<kHs>(const CscParams &, int, int, int, bool, hipStream_t);
-extern template hipError_t launch_csc_algo<kBl>(const CscParams &, int, int, int, bool, hipStream_t);
+template hipError_t launch_csc_algo<kChunk, false>(const CscParams &, int, int, int, bool, hipStream_t);
+extern template hipError_t launch_csc_algo<kSeq, false>(const CscParams &, int, int, int, bool, hipStream_t);
+extern template hipError_t launch_csc_algo<kHs, false>(const CscParams &, int, int, int, bool, hipStream_t);
+extern template hipError_t launch_csc_algo<kBl, false>(const CscParams &, int, int, int, bool, hipStream_t);
+extern template hipError_t launch_csc_algo<kChunk, true>(const CscParams &, int, int, int, bool, hipStream_t);
 
-// dBm, dCm: the channel tiles' partials of each (b, t, n); dA: the batch rows'.  Float64 sums in
+// dBm, dCm: the channel tiles' partials of each (b, t, n); dA: the batch rows' (and segments').  Float64 sums in
 // index order, the reads of 16 terms issued together.
 template <typename CT>
 __global__ void __launch_bounds__(kThreads) k_csc_fin(const CscParams p, int np) {
@@ -24,7 +25,7 @@ __global__ void __launch_bounds__(kThreads) k_csc_fin(const CscParams p, int np)
     vstore<CT>(o, b * o.s0 + t * o.s1 + n * o.s2, s);
   } else if (i < nBC + nA) {
     const int64_t j = i - nBC, n = j % p.N, d = j / p.N;
-    const double s = ordered_sum<16>((const double *)p.ws_dA + j, nA, p.B);
+    const double s = ordered_sum<16>((const double *)p.ws_dA + j, nA, p.B * p.nseg);
     vstore<CT>(p.dA, d * p.dA.s0 + n * p.dA.s1, (CT)s);
   }
 }
@@ -32,10 +33,12 @@ __global__ void __launch_bounds__(kThreads) k_csc_fin(const CscParams p, int np)
 hipError_t launch_csc(const CscParams &p, int algo, int dtype, int method, int np, bool bwd, hipStream_t s) {
   hipError_t e;
   switch (algo) {
-    case kSeq: e = launch_csc_algo<kSeq>(p, dtype, method, np, bwd, s); break;
-    case kHs: e = launch_csc_algo<kHs>(p, dtype, method, np, bwd, s); break;
-    case kBl: e = launch_csc_algo<kBl>(p, dtype, method, np, bwd, s); break;
-    default: e = launch_csc_algo<kChunk>(p, dtype, method, np, bwd, s);
+    case kSeq: e = launch_csc_algo<kSeq, false>(p, dtype, method, np, bwd, s); break;
+    case kHs: e = launch_csc_algo<kHs, false>(p, dtype, method, np, bwd, s); break;
+    case kBl: e = launch_csc_algo<kBl, false>(p, dtype, method, np, bwd, s); break;
+    default:
+      e = p.nseg > 1 ? launch_csc_algo<kChunk, true>(p, dtype, method, np, bwd, s)
+                     : launch_csc_algo<kChunk, false>(p, dtype, method, np, bwd, s);
   }
   if (e != hipSuccess || !bwd) return e;
   const int64_t n = p.B * p.L * 2 * np + p.D * p.N;

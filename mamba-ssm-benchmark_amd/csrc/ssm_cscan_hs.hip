@@ -3,5 +3,5 @@
 #include "ssm_cscan.hpp"
 
 namespace ssm {
-template hipError_t launch_csc_algo<kHs>(const CscParams &, int, int, int, bool, hipStream_t);
+template hipError_t launch_csc_algo<kHs, false>(const CscParams &, int, int, int, bool, hipStream_t);
 }  // namespace ssm

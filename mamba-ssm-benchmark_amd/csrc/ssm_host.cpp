@@ -408,6 +408,13 @@ py::tuple cscan_forward(const Tensor &x, const Tensor &delta, const Tensor &A, c
     ssm_cscan_args a = cscan_args(xb, db, A, Bm, Cm, h0, saved, i, n, algo, method);
     a.y = view(chans(y, 2, i, n));
     a.last = view(chans(last, 1, i, n));
+    SSM_BYTES(nb, ssm_cscan_fwd_workspace_bytes, ssm_cscan_check, a, "ssm_cscan_fwd");
+    Tensor ws;
+    if (nb) {
+      ws = bytes(nb, x);
+      a.workspace = ws.data_ptr();
+      a.workspace_bytes = nb;
+    }
     l.run("ssm_cscan_fwd", ssm_cscan_fwd, a, timer);
   }
   return py::make_tuple(y, last, Bm, Cm, out(saved));

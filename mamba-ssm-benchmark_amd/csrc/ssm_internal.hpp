@@ -205,11 +205,14 @@ __host__ __device__ constexpr int csc_tile(int algo, bool f64) { return algo == 
 struct CscParams {
   int64_t B, L, D, N;
   int64_t ntiles;  // channel tiles of the dB / dC partials
+  int nseg;        // time segments (chunked only; 1 otherwise) of seg_tiles time tiles each
+  int seg_tiles;
   KView x, dt, A, Bm, Cm, h0, y, last;
   KView saved;     // state entering each time tile: strides (b, tile, d), states consecutive
   KView dy, dlast, dx, ddelta, dA, dB, dC, dh0;
   void *ws_bc;     // (B, ntiles, L, 2, NP) state type: dB and dC partials over a tile's channels
-  void *ws_dA;     // (B, D, N) float64
+  void *ws_dA;     // (B, nseg, D, N) float64
+  void *ws_seg;    // nseg > 1: (2, B, nseg, D, N) state type, every segment's decay product and end value
 };
 hipError_t launch_csc(const CscParams &p, int algo, int dtype, int method, int np, bool bwd, hipStream_t s);
 

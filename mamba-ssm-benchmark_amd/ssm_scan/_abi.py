@@ -161,6 +161,7 @@ _SIGS = {
     "ssm_bwd_workspace_bytes": (c_i64, [ctypes.POINTER(BwdArgs)]),
     "ssm_lscan_workspace_bytes": (c_i64, [ctypes.POINTER(LscanArgs)]),
     "ssm_lscan_bwd_workspace_bytes": (c_i64, [ctypes.POINTER(LscanBwdArgs)]),
+    "ssm_cscan_fwd_workspace_bytes": (c_i64, [ctypes.POINTER(CscanArgs)]),
     "ssm_cscan_workspace_bytes": (c_i64, [ctypes.POINTER(CscanArgs)]),
     "ssm_disc_workspace_bytes": (c_i64, [ctypes.POINTER(DiscArgs)]),
     "ssm_conv_workspace_bytes": (c_i64, [ctypes.POINTER(ConvArgs)]),

@@ -463,3 +463,70 @@ def test_linear_scan_workspace_only_for_chunks(width, one_pass):
         for name in names:
             setattr(args, name, _abi.view(t))
         assert query(ctypes.byref(args)) == (0 if one_pass else -(-3 * 16 * width * 4 // 256) * 256)
+
+
+def _cscan_args(**kw):
+    B, L, D, N = kw.pop("shape", (1, 64, 4, 16))
+    t = torch.zeros(1)
+    a = _abi.CscanArgs()
+    a.batch, a.seqlen, a.dim, a.dstate, a.algo, a.method, a.dtype = B, L, D, N, 4, 0, 0
+    for name in ("x", "delta", "y", "dy", "dx", "ddelta"):
+        setattr(a, name, _abi.Tensor(t.data_ptr(), (ctypes.c_int64 * 3)(L * D, D, 1)))
+    for name in ("Bm", "Cm", "dBm", "dCm"):
+        setattr(a, name, _abi.Tensor(t.data_ptr(), (ctypes.c_int64 * 3)(L * N, N, 1)))
+    for name in ("A", "dA", "saved"):
+        setattr(a, name, _abi.Tensor(t.data_ptr(), (ctypes.c_int64 * 3)(N, 1, 0)))
+    a._keep = t
+    for k, v in kw.items():
+        setattr(a, k, v)
+    return a
+
+
+def test_composed_scan_refusals():
+    """What the composed scan's kernels cannot address or write is refused before any launch."""
+    lib = _abi.lib()
+    check = lambda a: _abi.check(lib.ssm_cscan_check(ctypes.byref(a)), "ssm_cscan")
+    bwd = lambda a: _abi.check(lib.ssm_cscan_bwd(ctypes.byref(a), None), "ssm_cscan_bwd")
+    check(_cscan_args())
+    for bad in (dict(algo=0), dict(algo=5), dict(dtype=1), dict(method=3), dict(shape=(0, 1, 1, 1)), dict(shape=(1, 1, 1, 65))):
+        with pytest.raises(ValueError):
+            check(_cscan_args(**bad))
+    a = _cscan_args(shape=(1, 64, 2, 16))
+    a.x.stride[1], a.x.stride[2] = 8000000, (1 << 29) - 1 - 63 * 8000000      # 64 steps end at 2^31 bytes
+    with pytest.raises(ValueError, match="strides"):
+        check(a)
+    a.x.stride[2] -= 1
+    check(a)
+    a.Bm.stride[1] = -16
+    with pytest.raises(ValueError, match="strides"):
+        check(a)
+    for name in ("saved", "dy", "dx", "ddelta", "dA", "dBm", "dCm"):
+        a = _cscan_args()
+        getattr(a, name).data = None
+        with pytest.raises(ValueError, match=name):
+            bwd(a)
+    a = _cscan_args()
+    a.dy.stride[2] = 1 << 29
+    with pytest.raises(ValueError, match="dy: strides"):
+        bwd(a)
+    a = _cscan_args()
+    a.dh0 = a.dA
+    with pytest.raises(ValueError, match="dh0"):
+        bwd(a)
+    a = _cscan_args()
+    need = lib.ssm_cscan_workspace_bytes(ctypes.byref(a))
+    a.workspace, a.workspace_bytes = a._keep.data_ptr(), need - 1
+    with pytest.raises(ValueError, match="workspace"):
+        bwd(a)
+
+
+@pytest.mark.parametrize("shape,algo,segments", [
+    ((1, 1023, 4, 16), 4, 4), ((1, 960, 4, 16), 4, 1), ((1, 1024, 4, 16), 3, 1), ((1, 16384, 4, 16), 4, 64),
+    ((2, 1088, 256, 16), 4, 2), ((1, 4096, 516, 16), 4, 1), ((1, 1089, 8, 4), 4, 4), ((64, 65536, 8, 16), 4, 2)])
+def test_composed_scan_segments(shape, algo, segments):
+    """Segments fill 256 workgroups, 4 tiles or more each, 64 at most, from 16 tiles on; the forward's
+    workspace holds two values per segment, channel and state."""
+    B, L, D, N = shape
+    a = _cscan_args(shape=shape, algo=algo)
+    want = 0 if segments == 1 else -(-2 * B * segments * D * N * 4 // 256) * 256
+    assert _abi.lib().ssm_cscan_fwd_workspace_bytes(ctypes.byref(a)) == want

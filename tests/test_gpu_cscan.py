@@ -6,6 +6,10 @@ the backward -- against the float64 oracle."""
 import pytest
 import torch
 
+import ctypes
+
+import ssm_scan
+from ssm_scan import _abi
 from ssm_scan import scan as S
 from test_gpu_scan import ALGOS, _oracle_sel, close, sel_inputs
 
@@ -126,12 +130,13 @@ def test_infinite_decay(scan, L):
 
 
 def test_operand_spans_up_to_2_gib():
-    """64 steps of a batch row may span up to 2^31 bytes, the last elements included."""
+    """64 steps of a batch row may span up to 2^31 bytes, the last elements included; a view that spans
+    more is copied."""
     ins, dy, dlast = _problem(1, 64, 3, 5, False, 21)
     x, delta, A, Bm, Cm, _ = (None if t is None else t.float().cuda() for t in ins)
-    store = torch.empty(1 << 29, device="cuda")
-    for s2 in (134217726, 134217727):   # one B for every step; its last state
-        Bs = store[:4 * s2 + 1].as_strided((1, 64, 5), (0, 0, s2))  # starts 32 and 16 bytes below 2^31
+    store = torch.empty((1 << 29) + 1, device="cuda")
+    for s2 in (134217726, 134217727, 134217728):   # one B for every step; its last state starts 32,
+        Bs = store[:4 * s2 + 1].as_strided((1, 64, 5), (0, 0, s2))  # 16 and 0 bytes below 2^31
         store[:4 * s2 + 1:s2] = Bm[0, 0]
         res = []
         for v in (Bm[:, :1].expand(1, 64, 5).contiguous(), Bs):
@@ -140,3 +145,51 @@ def test_operand_spans_up_to_2_gib():
             res.append((y, last, *torch.autograd.grad((y, last), leaves, (dy.float().cuda(), dlast.float().cuda()))))
         for got, want in zip(res[1], res[0]):
             assert torch.equal(got, want)
+
+
+# Time segments of the chunked algorithm (from 1024 steps, up to 256 workgroups): whole and ragged last
+# segments, segments shorter than their eight wavefronts' shares, the most segments, every padding
+SEGS = [(1, 1024, 3, 16), (2, 1025, 5, 12), (1, 1087, 9, 3), (3, 1100, 4, 33), (1, 16384, 1, 2), (1, 4200, 70, 16)]
+
+
+@pytest.mark.parametrize("shape", SEGS, ids=str)
+def test_time_segments_float64(shape):
+    for method, h0 in (("zoh", True), ("euler", False), ("bilinear", True)):
+        _run("chunked", method, *_problem(*shape, h0, 31), torch.float64)
+
+
+@pytest.mark.parametrize("shape", SEGS, ids=str)
+def test_time_segments_float32(shape):
+    _check_all("chunked", "zoh", *_problem(*shape, True, 32))
+
+
+def test_forward_without_workspace_walks_time_whole():
+    """ssm_cscan_fwd splits time only with its workspace; without, the sequence is one segment."""
+    ins, _, _ = _problem(1, 1300, 5, 16, True, 33)
+    x, delta, A, Bm, Cm, h0 = (t.float().cuda() for t in ins)
+    y, last = S.selective_scan(x, delta, A, Bm, Cm, h0, scan="chunked")
+    y1, last1 = torch.empty_like(y), torch.empty_like(last)
+    a = _abi.CscanArgs()
+    a.batch, a.seqlen, a.dim, a.dstate, a.algo = 1, 1300, 5, 16, 4
+    for name, t in (("x", x), ("delta", delta), ("A", A), ("Bm", Bm), ("Cm", Cm), ("h0", h0), ("y", y1), ("last", last1)):
+        setattr(a, name, _abi.view(t))
+    lib = _abi.lib()
+    assert lib.ssm_cscan_fwd_workspace_bytes(ctypes.byref(a)) > 0
+    _abi.check(lib.ssm_cscan_fwd(ctypes.byref(a), _abi.stream_handle(x.device)), "ssm_cscan_fwd")
+    _close_norm(y1, y.double().cpu(), "y")
+    _close_norm(last1, last.double().cpu(), "last")
+
+
+@pytest.mark.parametrize("scan", ["chunked", "sequential"])
+def test_backward_cuts_channels_to_its_workspace(scan):
+    """Without d_block a launch takes the channels whose partials fit 256 MiB: here 64 of 70."""
+    ins, dy, dlast = _problem(1, 8192, 70, 64, True, 34)
+    leaves = [t.float().cuda().requires_grad_() for t in ins]
+    out = []
+    for d_block in (None, 16):
+        y, last = S.selective_scan(*leaves, scan=scan, d_block=d_block)
+        with ssm_scan.KernelTimer() as t:
+            out.append(torch.autograd.grad((y, last), leaves, (dy.float().cuda(), dlast.float().cuda())))
+        assert len(t.records["ssm_cscan_bwd"]) == (2 if d_block is None else 5)
+    for name, got, ref in zip(("dx", "ddelta", "dA", "dB", "dC", "dh0"), *out):
+        _close_norm(got, ref.double().cpu(), name)
