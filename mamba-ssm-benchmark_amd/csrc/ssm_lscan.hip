@@ -113,12 +113,20 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
     nb[r] = ch.b_at(ch.t_of(pos));
     if constexpr (GRAD) nh[r] = ch.hprev_at(pos);
   };
-  // A row lane past the end of the sequence reads nothing, the one at the end at clamped positions.
-  // (One copy of the reads: a second one for whole tiles costs a short scan more than it saves.)
+  // A row lane past the end of the sequence reads nothing; at the end, one of consecutive steps reads at
+  // clamped positions (a second copy of the reads for whole tiles costs a short scan more than it
+  // saves), Hillis-Steele's skip theirs one by one (half a last tile of theirs lies past the end: L 80,
+  // 512 workgroups, forward 11.9 -> 11.0 us).  All conditions are uniform over the wavefront.
   auto fetch = [&](int base) {
     if (base + step(0) >= L) return;
 #pragma unroll
-    for (int r = 0; r < R; ++r) read(min(base + step(r), L - 1), r);
+    for (int r = 0; r < R; ++r) {
+      if constexpr (ALGO == kHs) {
+        if (base + step(r) < L) read(base + step(r), r);
+      } else {
+        read(min(base + step(r), L - 1), r);
+      }
+    }
   };
   fetch(0);
   int buf = 0;
@@ -133,13 +141,15 @@ __global__ void __launch_bounds__(RL * kScanMC) k_lscan_walk(const LscanParams P
     }
     if (base + T < L) fetch(base + T);
     CT hin;
-    tile_scan<CT, ALGO, RL, R>(X, a, b, carry, hin, tr, mi, buf);
+    auto emit = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int pos = base + step(r);
-      if (mval && pos < L) ch.template put<GRAD>(pos, b[r], hp[GRAD ? r : 0]);
-      if (GRAD && mval && pos + 1 == L) ch.put_dh0(b[r]);
-    }
+      for (int r = 0; r < R; ++r) {
+        const int pos = base + step(r);
+        if (mval && pos < L) ch.template put<GRAD>(pos, b[r], hp[GRAD ? r : 0]);
+        if (GRAD && mval && pos + 1 == L) ch.put_dh0(b[r]);
+      }
+    };
+    tile_scan<CT, ALGO, RL, R>(X, a, b, carry, hin, tr, mi, buf, emit);
   }
 }
 
@@ -312,7 +322,7 @@ __global__ void __launch_bounds__(256) k_lscan_chunk_scan(const LscanParams P) {
 // L 4096, forward + adjoint: 4 row lanes 165 + 349 us, 8 151 + 280, 16 164 + 338).  Two such
 // workgroups fit a CU (registers; Hillis-Steele: LDS), so from 512 workgroups on, Hillis-Steele past
 // it, 4 row lanes run in one round what 8 run in two (625 workgroups, hillis_steele, L 80 forward
-// 16 -> 11 us), until 1,024 fill two rounds either way (L 2048: 326 us with 8, 340 with 4); short
+// 16 -> 12 us), until 1,024 fill two rounds either way (L 2048: 326 us with 8, 340 with 4); short
 // sequences keep 4, whose workgroups hide each other's latencies (forward + adjoint, 1,024
 // workgroups, 8 -> 4: L 80 blelloch 46 -> 39, hillis_steele 45 -> 34; L 400 181 -> 178, 176 -> 169;
 // L 1000 424 -> 443, 433 -> 429).  A sequence of at most 4, 2 or 1 row lanes' steps takes no more
