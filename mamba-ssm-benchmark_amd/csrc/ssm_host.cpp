@@ -473,12 +473,10 @@ struct DecodePlan {
   std::vector<Block> blocks;
   Tensor head_w4;
   int64_t dm, dim, N, W, R, V;
-  int method;
-  double head_eps;
 
   DecodePlan(const std::vector<std::pair<std::vector<Tensor>, double>> &layers, Tensor head, int64_t dm_, int64_t dim_,
-             int64_t N_, int64_t W_, int64_t R_, int64_t V_, int method_, double eps)
-      : head_w4(std::move(head)), dm(dm_), dim(dim_), N(N_), W(W_), R(R_), V(V_), method(method_), head_eps(eps) {
+             int64_t N_, int64_t W_, int64_t R_, int64_t V_)
+      : head_w4(std::move(head)), dm(dm_), dim(dim_), N(N_), W(W_), R(R_), V(V_) {
     for (const auto &l : layers) {
       const auto &t = l.first;
       TORCH_CHECK_VALUE(t.size() == 9, "a decode block has 9 weights");
@@ -513,10 +511,8 @@ struct DecodePlan {
   void fill(ssm_decode_stack_args &a, int64_t B) const {
     memset(&a, 0, sizeof(a));
     a.batch = B; a.dim = dim; a.dstate = N; a.width = W; a.dt_rank = R; a.d_model = dm;
-    a.method = method;
     a.n_blocks = (int32_t)blocks.size();
     a.vocab = V;
-    a.head_eps = (float)head_eps;
   }
   int64_t workspace_bytes(int64_t B) const {
     ssm_decode_stack_args a;
@@ -529,9 +525,10 @@ struct DecodePlan {
     return ssm_decode_stack_status_offset(&a);
   }
 
-  // The whole token step in one call; returns the logits.
+  // The whole token step in one call; returns the logits.  The discretization and the final norm's eps
+  // are settings of the model, not weights: they come with each step.
   Tensor step(const Tensor &tok_, const std::vector<Tensor> &conv, const std::vector<Tensor> &ssm, const Tensor &embed,
-              const Tensor &ws) const {
+              const Tensor &ws, int method, double head_eps) const {
     for (const Tensor &c : conv)
       TORCH_CHECK_VALUE(c.scalar_type() == conv[0].scalar_type(),
                         "the stack path needs one conv state dtype for every block");
@@ -553,6 +550,8 @@ struct DecodePlan {
     }
     ssm_decode_stack_args a;
     fill(a, B);
+    a.method = method;
+    a.head_eps = (float)head_eps;
     a.conv_state_dtype = dtype_code(conv[0].scalar_type());
     a.blocks = k.data();
     a.u = (float *)u.data_ptr();
@@ -585,7 +584,7 @@ PYBIND11_MODULE(_ssmhost, m) {
   m.attr("ABI_VERSION") = SSM_ABI_VERSION;  // of the header the argument structs above were compiled from
   py::class_<DecodePlan>(m, "DecodePlan")
       .def(py::init<const std::vector<std::pair<std::vector<Tensor>, double>> &, Tensor, int64_t, int64_t, int64_t, int64_t,
-                    int64_t, int64_t, int, double>())
+                    int64_t, int64_t>())
       .def("check_states", torch::wrap_pybind_function(&DecodePlan::check_states))
       .def("workspace_bytes", &DecodePlan::workspace_bytes)
       .def("status_offset", &DecodePlan::status_offset)

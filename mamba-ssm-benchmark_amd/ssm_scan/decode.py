@@ -89,8 +89,7 @@ class FastDecoder:
             m, (V, dm) = self.layers[0]["mixer"], self.model.head.weight.shape
             names = ("w_in4", "conv_w", "conv_b", "x_proj_wt", "dt_proj_w", "dt_bias", "A_log", "Dskip", "w_out4")
             self.plan = _abi.host().DecodePlan([([L[k] for k in names], L["eps"]) for L in self.layers], head_w4, dm,
-                                               m.d_inner, m.d_state, m.d_conv, m.dt_rank, V,
-                                               METHODS[m.discretization], self.model.norm_f.eps)
+                                               m.d_inner, m.d_state, m.d_conv, m.dt_rank, V)
 
     def _layer(self, L, u, state):
         m = L["mixer"]
@@ -125,7 +124,8 @@ class FastDecoder:
             status = ws[off:off + 4].view(torch.int32)
             status.zero_()            # the library sets it, never clears it
             self._ws[key] = (ws, status)
-        return self.plan.step(tok, conv, ssm, self.model.embed.weight, self._ws[key][0])
+        return self.plan.step(tok, conv, ssm, self.model.embed.weight, self._ws[key][0],
+                              METHODS[self.layers[0]["mixer"].discretization], self.model.norm_f.eps)
 
     def _check(self, tok, states):
         """Host-side checks before any launch: the kernels size every state buffer from the
