@@ -747,6 +747,9 @@ int ssm_cscan_check(const ssm_cscan_args *a) {
   if (a->algo < SSM_SCAN_SEQUENTIAL || a->algo > SSM_SCAN_CHUNKED)
     return fail(SSM_EINVAL, "unknown scan algorithm %d (sequential=1 .. chunked=4)", a->algo);
   if (a->dtype != SSM_F32 && a->dtype != SSM_F64) return fail(SSM_EINVAL, "composed scans take float32 or float64");
+  // a grid row of fewer than 2^32 threads (8 wavefronts per channel tile): more would wrap, unreported
+  if (cdiv(a->dim, 64 / padded_n(a->dstate)) * 512 >= (1LL << 32))
+    return fail(SSM_EINVAL, "dim=%lld too large for one launch", (long long)a->dim);
   REQUIRE(a->x, "x");
   REQUIRE(a->delta, "delta");
   REQUIRE(a->A, "A");

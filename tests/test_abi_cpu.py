@@ -488,7 +488,8 @@ def test_composed_scan_refusals():
     check = lambda a: _abi.check(lib.ssm_cscan_check(ctypes.byref(a)), "ssm_cscan")
     bwd = lambda a: _abi.check(lib.ssm_cscan_bwd(ctypes.byref(a), None), "ssm_cscan_bwd")
     check(_cscan_args())
-    for bad in (dict(algo=0), dict(algo=5), dict(dtype=1), dict(method=3), dict(shape=(0, 1, 1, 1)), dict(shape=(1, 1, 1, 65))):
+    check(_cscan_args(shape=(1, 1, (1 << 23) - 1, 64)))
+    for bad in (dict(shape=(1, 1, 1 << 23, 64)), dict(algo=0), dict(algo=5), dict(dtype=1), dict(method=3), dict(shape=(0, 1, 1, 1)), dict(shape=(1, 1, 1, 65))):
         with pytest.raises(ValueError):
             check(_cscan_args(**bad))
     a = _cscan_args(shape=(1, 64, 2, 16))

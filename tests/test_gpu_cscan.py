@@ -193,3 +193,27 @@ def test_backward_cuts_channels_to_its_workspace(scan):
         assert len(t.records["ssm_cscan_bwd"]) == (2 if d_block is None else 5)
     for name, got, ref in zip(("dx", "ddelta", "dA", "dB", "dC", "dh0"), *out):
         _close_norm(got, ref.double().cpu(), name)
+
+
+def test_more_partials_than_a_launch_has_threads():
+    """2^25 steps of 33 states are 2^32 sums of dB and dC.  Only the last 64 steps carry anything."""
+    ins, dy, _ = _problem(1, 64, 1, 33, False, 35)
+    x, delta, A, Bm, Cm = (t.float().cuda() for t in ins[:5])
+    dy, L = dy.float().cuda(), 1 << 25
+
+    def tail(t):
+        out = torch.zeros(1, L, 1, device="cuda")
+        out[:, L - 64:] = t
+        return out
+
+    got = []
+    for ops, g in (((x, delta, Bm[:, :1].expand(1, 64, 33), Cm[:, :1].expand(1, 64, 33)), dy),
+                   ((tail(x), tail(delta), Bm[:, :1].expand(1, L, 33), Cm[:, :1].expand(1, L, 33)), tail(dy))):
+        leaves = [t.detach().requires_grad_() for t in (ops[0], ops[1], A, ops[2], ops[3])]
+        y, _ = S.selective_scan(*leaves, scan="chunked")
+        got.append(torch.autograd.grad(y, leaves, g))
+    small, large = got
+    for name, a, b in zip(("dx", "ddelta", "dB", "dC"), (small[i] for i in (0, 1, 3, 4)), (large[i] for i in (0, 1, 3, 4))):
+        _close_norm(b[:, L - 64:], a.double().cpu(), name)
+    _close_norm(large[2], small[2].double().cpu(), "dA")
+    assert not bool(large[3][:, :L - 64].any()) and not bool(large[4][:, :L - 64].any())
