@@ -189,7 +189,7 @@ template <typename CT, int CW>
 __global__ void __launch_bounds__(kConvFinThreads) k_conv_fin(const ConvParams p) {
   constexpr int G = kConvFinThreads / CW;
   __shared__ double red[G][CW];
-  const int l = threadIdx.x % CW, g = threadIdx.x / CW;
+  const int l = threadIdx.x, g = threadIdx.y;
   const int64_t cols = (p.W + 1) * p.D, e = (int64_t)blockIdx.x * CW + l, rows = p.B * p.nblk;
   double s = 0;
   if (e < cols && g < rows)
@@ -208,7 +208,8 @@ __global__ void __launch_bounds__(kConvFinThreads) k_conv_fin(const ConvParams p
 template <typename CT, int CW>
 static void conv_fin(const ConvParams &p, hipStream_t s) {
   const int64_t cols = (p.W + 1) * p.D;
-  hipLaunchKernelGGL((k_conv_fin<CT, CW>), dim3((unsigned)((cols + CW - 1) / CW)), dim3(kConvFinThreads), 0, s, p);
+  // (CW, row groups) threads: a grid row of 2^32 and more would wrap
+  hipLaunchKernelGGL((k_conv_fin<CT, CW>), dim3((unsigned)((cols + CW - 1) / CW)), dim3(CW, kConvFinThreads / CW), 0, s, p);
 }
 
 template <typename IT, int W>

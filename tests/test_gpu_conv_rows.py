@@ -92,3 +92,14 @@ def test_infinite_input_stays_within_its_taps(dev):
     x[:, 0] = float("inf")
     y = causal_conv1d(x, torch.ones(256, 4, device=dev), None, activation=False)
     assert bool(torch.isfinite(y[:, 4:130]).all()) and bool(torch.isinf(y[:, :4]).all())
+
+
+def test_more_columns_than_a_grid_row_has_threads(dev):
+    """2^26 channels x 4 taps and the bias: 16 threads for each of their sums are more than 2^32."""
+    D = 1 << 26
+    x = torch.arange(D, device=dev, dtype=torch.float32).remainder_(251.0).view(1, 1, D).requires_grad_()
+    w, b = torch.ones(D, 4, device=dev).requires_grad_(), torch.zeros(D, device=dev).requires_grad_()
+    y = causal_conv1d(x, w, b, activation=False)
+    dw, db = torch.autograd.grad(y, (w, b), torch.full_like(y, 2.0))
+    assert torch.equal(dw[:, 3], 2 * x.detach().view(D)) and not bool(dw[:, :3].any())
+    assert bool((db == 2).all())
