@@ -38,6 +38,8 @@
 // chunked 154 + 281 us (in three launches with a separate adjoint epilogue 295 + 570), blelloch
 // 151 + 284 (with 4 row lanes 200 + 484), hillis_steele 184 + 290 (237 + 511), sequential 149 +
 // 283 (one wavefront per workgroup 185 + 467).
+#include <algorithm>
+
 #include "ssm_device.hpp"
 #include "ssm_dpp.hpp"
 #include "ssm_internal.hpp"
@@ -328,7 +330,21 @@ __global__ void __launch_bounds__(256) k_lscan_chunk_scan(const LscanParams P) {
 // L 1000 424 -> 443, 433 -> 429).  A sequence of at most 4, 2 or 1 row lanes' steps takes no more
 // than these (sequential, 1,024 workgroups, 8 -> this: L 64 44 -> 26, L 16 39 -> 11).
 template <typename CT, int ALGO, bool GRAD>
-static hipError_t launch_walk(const LscanParams &P, hipStream_t s) {
+static hipError_t launch_walk(const LscanParams &all, hipStream_t s) {
+  // A grid row holds fewer than 2^32 threads (more would wrap, unreported): wider scans take several.
+  constexpr int64_t kMaxM = 1LL << 28;
+  if (all.M > kMaxM) {
+    for (int64_t m = 0; m < all.M; m += kMaxM) {
+      LscanParams P = all;
+      P.M = std::min(all.M - m, kMaxM);
+      for (KView *v : {&P.a, &P.b, &P.h, &P.hf, &P.da}) v->p = v->p ? (CT *)v->p + m * v->s2 : nullptr;
+      for (KView *v : {&P.h0, &P.h0f, &P.dh0}) v->p = v->p ? (CT *)v->p + m * v->s1 : nullptr;
+      const hipError_t e = launch_walk<CT, ALGO, GRAD>(P, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  const LscanParams &P = all;
   const dim3 tiles((unsigned)((P.M + kScanMC - 1) / kScanMC), (unsigned)P.B);
   const int64_t g = lscan_groups(P.B, P.M);
   constexpr int R = scan_rows(ALGO);

@@ -85,3 +85,20 @@ def test_chunk_sizes_on_both_sides_of_the_one_pass_rule(M, chunk):
     da_atol = max(1e-5, 16 * 2.0 ** -24 * refs[0].abs().max().item() * refs[2].abs().max().item())  # as above
     for name, got, ref in zip(("h", "da", "db", "dh0"), (h.detach(), *torch.autograd.grad(h, leaves, dh)), refs):
         close(got, ref, name=name, **({"atol": da_atol} if name == "da" else {}))
+
+
+@pytest.mark.parametrize("algo", ["sequential", "blelloch"])
+def test_width_cut_into_launches(algo):
+    """2^29 recurrences of 8 wavefronts per 64 are 2^32 threads, more than a launch has; they are walked in
+    several, 2^28 each: columns around the cuts, with h0."""
+    L, M = 3, (1 << 29) + 65
+    a = torch.full((1, 1, 1), 0.5, device="cuda").expand(1, L, M)
+    b = torch.arange(M, device="cuda", dtype=torch.float32).remainder_(127.0).expand(1, L, M)
+    h0 = (torch.arange(M, device="cuda", dtype=torch.float32).remainder_(61.0) - 30).view(1, M).requires_grad_()
+    ad = a.detach().requires_grad_()
+    h = S.LinearScanFn.apply(ad, b, h0, S._SCAN_ALGO[algo], 0, False)
+    da, dh0 = torch.autograd.grad(h, (ad, h0), torch.ones(1, 1, 1, device="cuda").expand(1, L, M))
+    cols = torch.cat([torch.arange(70), torch.arange((1 << 28) - 70, (1 << 28) + 70), torch.arange((1 << 29) - 70, M)]).cuda()
+    refs = _ref(a[..., cols], b[..., cols], h0.detach()[:, cols], torch.ones(1, L, len(cols), device="cuda"), False)
+    for got, ref in ((h.detach()[..., cols], refs[0]), (da[..., cols], refs[1]), (dh0[:, cols], refs[3])):
+        torch.testing.assert_close(got.double(), ref, rtol=1e-6, atol=1e-6)   # a few float32 roundings
