@@ -3,7 +3,8 @@
 // contracts, where the reference materializes a, b, h, their gradients and the adjoint.
 //
 // A workgroup owns 64 / NP channels x NP states (one recurrence per lane) of one batch row and walks
-// time (with the chunked algorithm, few workgroups and a long sequence: one segment of it) in tiles of RL row lanes (wavefronts) x R steps.  Forward: a tile's x, delta, B, C are read
+// time in tiles of RL row lanes (wavefronts) x R steps; with the chunked algorithm, few workgroups and
+// a long sequence it walks one segment of time (k_csc_sum).  Forward: a tile's x, delta, B, C are read
 // while the previous tile is scanned, a and b are formed in registers as k_disc_fwd forms them, and
 // y = sum_n C h is summed over the state lanes before it is stored.  It saves the state entering
 // every tile.  Backward, from the last tile to the first: the tile's states are recomputed from the
@@ -21,9 +22,10 @@
 // Bound: VALU issue (24 + 66 instructions per (b, t, d, n) element) and the latency of a tile's LDS
 // exchanges, not HBM: the materialized form moved 6-8 (B, L, D, N) tensors forward and 19 in a
 // training step, this moves 2 / CW of one (the dB / dC partials, CW = 64 / NP) twice.  B2 L2048
-// D512 N16 float32, chunked, forward + backward: 41 + 89 + 11 us of kernels, 26 launches of 1,030 us
-// before.  8 steps per lane keep a backward lane's tile in registers (200 VGPRs: two wavefronts per
-// SIMD); 8 row lanes give the 256 workgroups of that shape 2 wavefronts per SIMD.
+// D512 N16 float32, chunked, forward + backward: 41 + 87 + 11 us of kernels, 26 launches of 1,030 us
+// before (sequential 51 + 97, Blelloch 47 + 86, Hillis-Steele 67 + 179).  8 steps per lane keep a
+// backward lane's tile in registers (166 VGPRs: one workgroup per CU); 8 row lanes give the 256
+// workgroups of that shape 2 wavefronts per SIMD.
 #pragma once
 
 #include "ssm_device.hpp"
@@ -162,7 +164,7 @@ template <typename CT, int ALGO> constexpr int cs_rows() { return csc_tile(ALGO,
 // A wavefront's R steps x COLS channels (or states) of a (B, L, C) operand: read one element per lane
 // along whichever axis has unit stride, and laid out in LDS as rows of R steps that a lane reads
 // with 16-byte loads.  (A read per lane and step -- 4-5 R loads per tile of 64 or fewer distinct
-// bytes each -- kept the address units 54 % busy: 62 + 121 us where this takes 41 + 89,
+// bytes each -- kept the address units 54 % busy: 62 + 121 us where this takes 41 + 87,
 // at the shape above.)
 template <typename CT, int R, int COLS>
 struct TileIn {

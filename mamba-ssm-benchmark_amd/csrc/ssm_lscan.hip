@@ -35,9 +35,9 @@
 // Bound: HBM.  3 (adjoint: 5) tensors of s B L M bytes move once.  What a workgroup keeps in
 // flight sets the rate: 8 row lanes x 16 steps x 2-3 tensors x 256 bytes.  At (B, L, M) = (2,
 // 4096, 8192) float32, forward + adjoint, where a copy of the same bytes takes 155 + 259 us:
-// chunked 154 + 281 us (in three launches with a separate adjoint epilogue 295 + 570), blelloch
-// 151 + 284 (with 4 row lanes 200 + 484), hillis_steele 184 + 290 (237 + 511), sequential 149 +
-// 283 (one wavefront per workgroup 185 + 467).
+// chunked 159 + 257 us (in three launches with a separate adjoint epilogue 295 + 570), blelloch
+// 159 + 256 (with 4 row lanes 200 + 484), hillis_steele 181 + 269 (237 + 511), sequential 156 +
+// 256 (one wavefront per workgroup 185 + 467).
 #include <algorithm>
 
 #include "ssm_device.hpp"

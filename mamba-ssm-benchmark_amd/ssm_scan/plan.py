@@ -1,7 +1,8 @@
 """The reference's integer planning functions, computed by the engine library (exact integers).
 
   default_chunk   models/scan.py:138-139
-  blocks          models/scan.py:185-190 (channel tiles of SelectiveScanFn)
+  blocks          models/scan.py:185-190 (the reference's channel tiles of SelectiveScanFn; the
+                  engine's composed scan needs none and cuts channels only by d_block or workspace)
   block_d         kernels/triton_scan.py:245-250
   bwd_tile        kernels/triton_scan.py:305
   resolve_scan    models/scan.py:286-287 with _triton_ok :305-314 (the selected algorithm)

@@ -38,7 +38,7 @@ def default_chunk(L):
 
 
 def _blocks(shape_bld, N, d_block):
-    """Channel tiles of SelectiveScanFn (models/scan.py:185-190)."""
+    """The reference's channel tiles of SelectiveScanFn (models/scan.py:185-190); here they plan nothing."""
     return plan.blocks(shape_bld, N, d_block)
 
 
@@ -220,8 +220,9 @@ class SelectiveScanFn(torch.autograd.Function):
     entering every time tile.  The backward recomputes the states tile by tile, runs the adjoint
     scan lambda_t = g_t + a_{t+1} lambda_{t+1} with the same algorithm and maps (da, db) =
     (lambda h_{t-1}, lambda) back through the discretization, in channel tiles of d_block (default:
-    as many channels as keep the workspace within 256 MiB).  chunk_size is the chunk of the linear scan over materialized
-    tensors; here a chunk is a wavefront's part of a time tile."""
+    as many channels as keep the workspace within 256 MiB).  d_block bounds that workspace only (the
+    forward has none to speak of), and chunk_size changes nothing: it is the chunk of a linear scan over
+    materialized tensors, where here a chunk is a wavefront's part of a time tile."""
 
     @staticmethod
     def forward(ctx, x, delta, A, Bm, Cm, h0, method, scan_name, d_block, chunk_size):
